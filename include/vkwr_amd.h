@@ -337,11 +337,17 @@ typedef struct vkwr_gemm_problem {
   const uint16_t* v0;
 } vkwr_gemm_problem;
 
-/* Bytes of device workspace vkwr_gemm_f16 needs for this batch (fp32 partial
- * sums: K splits of small-M problems, or the k-parts of a large-M batch's last
- * round of 256x256 tiles; 0 when nothing is split), or -1 on invalid arguments.
- * The plan depends on the current device's CU count: ask on that device. */
+/* Bytes of device workspace vkwr_gemm_f16 wants for this batch (fp32 partial
+ * sums: K splits of small-M and mid-size problems, or the k-parts of a large-M batch's
+ * last round of 256x256 tiles; 0 when nothing is split), or -1 on invalid arguments.
+ * The plan depends on the current device's CU count: ask on that device.  (Where only the
+ * mid-size path would split, vkwr_gemm_f16 with less runs that path in fewer parts.) */
 VKWR_EXPORT int64_t vkwr_gemm_f16_workspace_bytes(int n_problems, const vkwr_gemm_problem* problems);
+
+/* The largest workspace the batch needs when every problem's m is replaced by the same row
+ * count, over 1 .. problems[0].m (the plan is not monotone in the row count): for buffers
+ * that serve every batch size up to a limit.  -1 on invalid arguments. */
+VKWR_EXPORT int64_t vkwr_gemm_f16_workspace_bytes_upto(int n_problems, const vkwr_gemm_problem* problems);
 
 /* Runs 1..8 independent GEMMs in one launch on the gfx950 matrix cores.
  * `problems` is a host array; `workspace` is device memory of at least

@@ -68,6 +68,7 @@ def _sig(name, args, res=_i):
 _LIB.vkwr_last_error.restype = ctypes.c_char_p
 _gemm = _sig("vkwr_gemm_f16", [_i, ctypes.POINTER(GemmProblem), _p, _i64, _p])
 _gemm_ws = _sig("vkwr_gemm_f16_workspace_bytes", [_i, ctypes.POINTER(GemmProblem)], _i64)
+_gemm_ws_upto = _sig("vkwr_gemm_f16_workspace_bytes_upto", [_i, ctypes.POINTER(GemmProblem)], _i64)
 _ln_mix = _sig("vkwr_add_layer_norm_mix_f16",
                [_i64, _i, _p, _p, _p, _p, _p, _i, ctypes.POINTER(_p), _f, _p, ctypes.POINTER(_p), _p, _p, _i64, _i64,
                 _p])
@@ -167,18 +168,12 @@ def gemm_workspace_bytes_upto(problems):
     replaced by the same R, over R = 1 .. the problems' common row count.  The GEMM plan (tile
     shape, K splits, the large-M kernel's split last round) is not monotone in the row count,
     so a buffer sized for the largest batch, or for a few row counts, can fall short at others."""
-    arr = _arr(problems)
     rows = {int(p.m) for p in problems}
     assert len(rows) == 1, f"problems must share the row count (got {sorted(rows)})"
-    best = 0
-    for m in range(1, rows.pop() + 1):
-        for i in range(len(problems)):
-            arr[i].m = m
-        n = _gemm_ws(len(problems), arr)
-        if n < 0:
-            raise RuntimeError(f"vkwr_gemm_f16_workspace_bytes: {_LIB.vkwr_last_error().decode()}")
-        best = max(best, n)
-    return best
+    n = _gemm_ws_upto(len(problems), _arr(problems))
+    if n < 0:
+        raise RuntimeError(f"vkwr_gemm_f16_workspace_bytes_upto: {_LIB.vkwr_last_error().decode()}")
+    return n
 
 
 def gemm(problems, workspace):

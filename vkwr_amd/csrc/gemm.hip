@@ -6,7 +6,12 @@
 // into BM x BN output tiles and optionally into K splits; the flat workgroup
 // index walks problem -> M tile -> N tile -> K split.
 //
-// Tile loop: 256 lanes (4 waves in a WM x WN grid), K advanced 32 at a time.
+// Five kernel families, picked per launch by size, layout and alignment (build_batch, mid_choose):
+// GEMV-shaped (M <= 4), small M (gemm_rm_kernel, up to 128 rows), mid-size (gemm_mid_kernel), large
+// M (gemm_big_kernel), and the row-major tile kernel below for operands that are not 16-byte
+// aligned or whose K or N is no multiple of 8.
+//
+// Row-major tile loop: 256 lanes (4 waves in a WM x WN grid), K advanced 32 at a time.
 // Each stage moves an A tile (BM x 32) and a B tile (BN x 32, stored k-inner)
 // global -> VGPRs -> LDS, double buffered: the next stage's global loads are
 // issued before the current stage's MFMAs, and one barrier per stage separates
@@ -959,6 +964,433 @@ __global__ __launch_bounds__(256) void gemm_big_fixup_kernel(Batch bt, BigPlan p
   }
 }
 
+// ---- mid-size path: whole-K or K-split tiles of BM x BN fed through a ring of LDS stages.
+//
+// Takes the batches between the two paths below and above it: more rows than the small-M path
+// holds, too few 256-row tiles for the large-M path to fill the CUs, [K,N] weights, A-operand
+// activations, or K not a multiple of 64.  256 lanes = 4 waves in a 2x2 grid, each wave a
+// (BM/2) x (BN/2) sub-tile of 32x32 blocks.  K advances 64 per stage through a ring of NBUF LDS
+// buffers filled by the DMA form of the vector load, so that NBUF - 1 stages are in flight
+// while one is computed on: at these sizes a CU holds one or two workgroups and a stage of
+// matrix work (0.2-0.4 us) is shorter than a trip to memory.  One barrier per stage, placed
+// before the last k16 group's products: after it the stage's buffer is free (its fragments are
+// in registers) and is refilled, and the next stage has landed in every wave's view.
+//
+// A and [N,K] B rows are staged 64 k = 128 bytes wide with the swizzle of the large-M path; a
+// [K,N] B is staged as 64 k rows of BN columns and its fragments read with the transposing
+// LDS read, chunk c of k row r at c ^ 4 (r % 4) (BN >= 128) or c ^ 4 ((r / 2) % 2) (BN = 64), so
+// that the 4 rows x 64 bytes that 32 lanes read at once fall into different banks.
+// The last stage of a K that is no multiple of 64 is read clamped and its excess zeroed in LDS,
+// in both operands, before the barrier that publishes it.
+// Accumulation runs over k16 chunks in increasing order from zero, as in gemm_kernel.
+//
+// What bounds it: a 128 x 128 stage moves 32 KiB into LDS and 64 KiB out of it for 512 clocks of
+// matrix work per SIMD, and takes ~0.5 us with every CU busy (0.21 at the matrix peak); K = 8192,
+// M = N = 2048 runs in 69 us (1.0 PFLOP/s; large-M kernel 79, [K,N] row-major tiles 462).  With
+// the whole DMA of a stage issued in one group instead of a quarter in each it took 85 us: the
+// texture path takes a 1 KiB instruction every 16 clocks and held up the products behind it.
+constexpr int kMidBK = 64;
+
+__device__ __forceinline__ constexpr int mid_st_row(int tn) { return 32 * tn + 4; }  // floats per staged output row
+
+// Stores a wave's (32 TM) x (32 TN) accumulators: epilogue kEpi and fp16, or (kPartial) fp32
+// sums to the K part's plane.  32-row strips go through the wave's own LDS staging area, so
+// that each lane finishes 8 consecutive columns.
+template <int TM, int TN, bool kPartial, int kEpi>
+__device__ __forceinline__ void mid_store(float* st, const Prob& P, const fv16 (&acc)[TM][TN], int row0, int col0,
+                                          int split, int lane) {
+  constexpr int kRow = mid_st_row(TN), kLpr = 4 * TN, kRows = 64 / kLpr;  // lanes per row, rows per pass
+  typedef _Float16 __attribute__((address_space(1)))* gptr;
+  typedef const _Float16 __attribute__((address_space(1)))* gcptr;
+  typedef float __attribute__((address_space(1)))* gfptr;
+  const int lr = lane & 31, lh = lane >> 5;
+  int pm = P.m, pn = P.n, pvec = P.vec_out;
+  gptr pc = (gptr)P.c;
+  gcptr pv = (gcptr)P.v, pvf = (gcptr)P.vf, pv0 = (gcptr)P.v0;
+  gfptr pws = (gfptr)(P.ws + (kPartial ? (int64_t)split * P.m * P.n : 0));
+  asm("" : "+s"(pm), "+s"(pn), "+s"(pvec), "+s"(pc), "+s"(pv), "+s"(pvf), "+s"(pv0), "+s"(pws));
+  const int c8 = 8 * (lane % kLpr), rl = lane / kLpr, col = col0 + c8;
+  const bool cin = col < pn;
+  constexpr bool kVres = kEpi == VKWR_GEMM_EPI_VALUE_RESIDUAL;
+  constexpr bool kCol = !kPartial && (kVres || kEpi == VKWR_GEMM_EPI_BIAS);
+  hv8 v0{};
+  if constexpr (kCol) v0 = *reinterpret_cast<const __attribute__((address_space(1))) hv8*>(pv0 + (cin ? col : 0));
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) st[(8 * (r >> 2) + 4 * lh + (r & 3)) * kRow + 32 * j + lr] = acc[i][j][r];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int h = 0; h < 32 / kRows; ++h) {
+      const int row = row0 + 32 * i + h * kRows + rl;
+      const float* sp = st + (h * kRows + rl) * kRow + c8;
+      const f4 lo = *reinterpret_cast<const f4*>(sp), hi = *reinterpret_cast<const f4*>(sp + 4);
+      if (row >= pm || !cin) continue;
+      const int64_t idx = (int64_t)row * pn + col;
+      const float s8[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      if constexpr (kPartial) {
+        if (pvec) {
+          *reinterpret_cast<__attribute__((address_space(1))) f4*>(pws + idx) = lo;
+          *reinterpret_cast<__attribute__((address_space(1))) f4*>(pws + idx + 4) = hi;
+        } else {  // a workspace that is not 16-byte aligned
+#pragma unroll
+          for (int e = 0; e < 8; ++e) pws[idx + e] = s8[e];
+        }
+      } else {
+        hv8 o, vv{}, vf{};
+        if constexpr (kVres) {
+          vv = *reinterpret_cast<const __attribute__((address_space(1))) hv8*>(pv + idx);
+          vf = *reinterpret_cast<const __attribute__((address_space(1))) hv8*>(pvf + idx);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float y;
+          if constexpr (kVres) y = __builtin_fmaf((float)vf[e] - (float)vv[e], sigmoidf((float)v0[e] + s8[e]), (float)vv[e]);
+          else if constexpr (kEpi == VKWR_GEMM_EPI_BIAS) y = s8[e] + (float)v0[e];
+          else y = big_epilogue<kEpi>(P, s8[e], row, col + e);
+          asm volatile("" : "+v"(y));  // round in fp32, then to fp16 (no fused mixed-precision op)
+          o[e] = (_Float16)y;
+        }
+        *reinterpret_cast<__attribute__((address_space(1))) hv8*>(pc + idx) = o;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <int BM, int BN, int NBUF, bool kKN, bool kAct>
+__global__ __launch_bounds__(256) void gemm_mid_kernel(Batch bt, int wgs) {
+  constexpr int TM = BM / 64, TN = BN / 64;                      // 32x32 blocks per wave
+  constexpr int kA = BM * kMidBK, kB = BN * kMidBK, kStage = kA + kB;  // halves
+  constexpr int NA = BM / 32, NB = BN / 32, ND = NA + NB;        // DMA instructions per wave and stage
+  constexpr int kBc = BN / 8;                                    // [K,N]: 16-byte chunks per k row
+  static_assert(NBUF == 3 || NBUF == 4, "ring of 3 or 4 stages");
+  static_assert(4 * 32 * mid_st_row(TN) * 4 <= NBUF * kStage * 2, "output staging must fit the ring");
+  __shared__ __attribute__((aligned(1024))) _Float16 sm[NBUF * kStage];
+
+  // ---- problem, K part and tile (workgroup-uniform).  XCD-contiguous; a batch of unequal K
+  // (xbal, longest first) deals its tiles out round robin instead, so that no XCD is left with
+  // the long ones.
+  const int L = bt.xbal ? (int)blockIdx.x : xcd_contiguous(blockIdx.x, wgs);
+  int pi = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxProblems; ++i)
+    if (i < bt.n && L >= bt.p[i].tile_begin) pi = i;
+  const Prob& P = bt.p[pi];
+  {
+    // every field in one round of kernel-argument loads, before the first branch
+    const _Float16 *fa = P.a, *fb = P.b;
+    const int f0 = P.m, f1 = P.n, f2 = P.k, f3 = P.a_act, f4_ = P.epi, f6 = P.tiles_m, f7 = P.tiles_n, f8 = P.splits,
+              f9 = P.k_per_split, f10 = P.tile_begin;
+    asm volatile("" ::"s"(fa), "s"(fb), "s"(f0), "s"(f1), "s"(f2), "s"(f3), "s"(f4_), "s"(f6), "s"(f7), "s"(f8),
+                 "s"(f9), "s"(f10));
+  }
+  const int ntiles = P.tiles_m * P.tiles_n;
+  const int lt0 = L - P.tile_begin, split = lt0 / ntiles, lt = lt0 - split * ntiles;
+  constexpr int kGroup = 4;  // tile rows walked together (column-major inside a group)
+  const int per = kGroup * P.tiles_n, grp = lt / per, in = lt - grp * per;
+  const int g0 = grp * kGroup, gs = min(kGroup, P.tiles_m - g0);
+  const int m0 = (g0 + in % gs) * BM, n0 = (in / gs) * BN;
+  const int M = P.m, N = P.n, K = P.k, a_act = kAct ? P.a_act : VKWR_GEMM_ACT_NONE;
+  const int kbeg = split * P.k_per_split, klen = min(K - kbeg, P.k_per_split);
+  const int ns = (klen + kMidBK - 1) / kMidBK;
+  const bool ragged = klen % kMidBK != 0;
+
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wm = w >> 1, wn = w & 1;
+  const int lr = lane & 31, lh = lane >> 5;
+
+  // ---- staging: DMA instruction j of wave w fills slots j * 256 + w * 64 + lane of an operand
+  auto brow_sw = [](int r) { return BN >= 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
+  uint32_t ao[NA], bo[NB];
+#pragma unroll
+  for (int j = 0; j < NA; ++j) {
+    const int sl = j * 256 + tid, row = sl >> 3, c = (sl & 7) ^ ((row >> 1) & 7);
+    ao[j] = (uint32_t)(((int64_t)min(m0 + row, M - 1) * K + c * 8) * 2);
+  }
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int sl = j * 256 + tid;
+    if constexpr (kKN) {
+      const int r = sl / kBc, c = (sl % kBc) ^ brow_sw(r);
+      bo[j] = (uint32_t)(((int64_t)r * N + min(n0 + c * 8, N - 8)) * 2);
+    } else {
+      const int row = sl >> 3, c = (sl & 7) ^ ((row >> 1) & 7);
+      bo[j] = (uint32_t)(((int64_t)min(n0 + row, N - 1) * K + c * 8) * 2);
+    }
+  }
+  const _Float16* const pa = (const _Float16*)uniform_ptr(P.a);
+  const _Float16* const pb = (const _Float16*)uniform_ptr(P.b);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&sm[0] + w * 1024);
+  // DMA instruction d (0 .. ND - 1) of a stage: ab / bb its operands' first k (uniform), la the
+  // LDS address of its buffer; kTail: the part's last, ragged stage, chunks (rows) past its end
+  // read clamped to the last one
+  auto dma_one = [&](auto tail_tag, int d, const void* ab, const void* bb, uint32_t la, int left)
+                     __attribute__((always_inline)) {
+    constexpr bool kTail = decltype(tail_tag)::value;
+    const int j = d < NA ? d : d - NA;
+    uint32_t o = d < NA ? ao[d < NA ? d : 0] : bo[d < NA ? 0 : j];
+    if constexpr (kTail) {
+      if (kKN && d >= NA) {
+        o -= (uint32_t)(max((j * 256 + tid) / kBc - (left - 1), 0) * (int64_t)N * 2);
+      } else {
+        const int sl = j * 256 + tid, c = (sl & 7) ^ (((sl >> 3) >> 1) & 7);
+        o -= (uint32_t)(max(c * 8 - (left - 8), 0) * 2);
+      }
+    }
+    dma16_m0(d < NA ? ab : bb, o, la + (d < NA ? 0 : kA * 2) + j * 4096);
+  };
+  struct Src {
+    const void *a, *b;
+    uint32_t la;
+    int left;
+  };
+  auto src_of = [&](int buf, int st) __attribute__((always_inline)) {
+    const int k0 = kbeg + st * kMidBK;
+    return Src{uniform_ptr(pa + k0), uniform_ptr(kKN ? pb + (int64_t)k0 * N : pb + k0),
+               lds0 + (uint32_t)(buf * kStage * 2), klen - st * kMidBK};
+  };
+  auto dma_stage = [&](int buf, int st) __attribute__((always_inline)) {
+    const Src f = src_of(buf, st);
+    if (ragged && st == ns - 1) {
+#pragma unroll
+      for (int d = 0; d < ND; ++d) dma_one(std::true_type{}, d, f.a, f.b, f.la, f.left);
+    } else {
+#pragma unroll
+      for (int d = 0; d < ND; ++d) dma_one(std::false_type{}, d, f.a, f.b, f.la, f.left);
+    }
+  };
+  // applies the A activation to what this thread staged (its own DMA of the stage has landed), once
+  // per element and tile; on the fragments every wave column would repeat it
+  auto act_stage = [&](int buf) __attribute__((always_inline)) {
+    if (kAct && a_act != VKWR_GEMM_ACT_NONE) {
+#pragma unroll
+      for (int j = 0; j < NA; ++j) {
+        hv8* const p = reinterpret_cast<hv8*>(sm + buf * kStage + (j * 256 + tid) * 8);
+        hv8 v = *p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (_Float16)act_in((float)v[e], a_act);
+        *p = v;
+      }
+    }
+  };
+  // zeroes what this thread staged past the end of K (its own DMA of the stage has landed)
+  auto zero_tail = [&](int buf) __attribute__((always_inline)) {
+    _Float16* const sa = sm + buf * kStage;
+    const int left = klen - (ns - 1) * kMidBK;
+#pragma unroll
+    for (int j = 0; j < NA; ++j) {
+      const int sl = j * 256 + tid, c = (sl & 7) ^ (((sl >> 3) >> 1) & 7);
+      if (c * 8 >= left) *reinterpret_cast<hv8*>(sa + sl * 8) = hv8{};
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int sl = j * 256 + tid;
+      const bool past = kKN ? sl / kBc >= left : ((sl & 7) ^ (((sl >> 3) >> 1) & 7)) * 8 >= left;
+      if (past) *reinterpret_cast<hv8*>(sa + kA + sl * 8) = hv8{};
+    }
+  };
+
+  // ---- fragments of k16 group kk (offsets in halves)
+  int fao[4], fbo[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    const int sw = ((2 * kk + lh) ^ ((lr >> 1) & 7)) * 8;
+    fao[kk] = (wm * (BM / 2) + lr) * kMidBK + sw;
+    if constexpr (!kKN) fbo[kk] = kA + (wn * (BN / 2) + lr) * kMidBK + sw;
+  }
+  const int qg = lane >> 4, ql = lane & 15;  // [K,N]: 16-lane group of the transposing read
+  if constexpr (kKN) {
+    static_assert(TN <= 4, "one offset per column block");
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = wn * (BN / 2) + 32 * j + 16 * (qg & 1) + 4 * (ql & 3), r = 8 * (qg >> 1) + (ql >> 2);
+      fbo[j] = kA + r * BN + (((n >> 3) ^ brow_sw(r)) * 8) + (n & 7);
+    }
+  }
+  hv8 fa[2][TM], fb[2][TN];
+  auto fread = [&](int buf, int kk, int set) __attribute__((always_inline)) {
+    const _Float16* const s = sm + buf * kStage;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      fa[set][i] = *reinterpret_cast<const hv8*>(s + fao[kk] + 32 * i * kMidBK);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (kKN) {
+        typedef short sv4 __attribute__((ext_vector_type(4)));
+        typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
+        sv4 part[2];
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+          part[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (VK_LDS sv4*)((VK_LDS _Float16*)s + fbo[j] + (16 * kk + 4 * hf) * BN));
+        fb[set][j] = __builtin_shufflevector(__builtin_bit_cast(hv4, part[0]), __builtin_bit_cast(hv4, part[1]), 0, 1,
+                                             2, 3, 4, 5, 6, 7);
+      } else {
+        fb[set][j] = *reinterpret_cast<const hv8*>(s + fbo[kk] + 32 * j * kMidBK);
+      }
+    }
+  };
+  fv16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+  // the products of one k16 group, with quarter q of the DMA of a stage between them (kDma: 0
+  // none, 1 a whole stage, 2 the ragged last one): the texture path takes 64 bytes a clock, a
+  // stage's DMA as long as its products, so it is spread over all four groups
+  auto mfma = [&](int set, auto dma_tag, int q, const Src& f) __attribute__((always_inline)) {
+    constexpr int kDma = decltype(dma_tag)::value;
+    const int d0 = q * ND / 4, d1 = (q + 1) * ND / 4;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[set][i], fb[set][j], acc[i][j], 0, 0, 0);
+        if constexpr (kDma != 0) {
+          const int p = i * TN + j;
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            if (d >= d0 && d < d1 && (d - d0) * TM * TN / (d1 - d0) == p)
+              dma_one(std::integral_constant<bool, kDma == 2>{}, d, f.a, f.b, f.la, f.left);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+  };
+  // Waits until all but the newest `n` DMA instructions of this wave have landed.
+  auto wait_dma = [&](auto n) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory");
+  };
+  auto whole = [](auto n) { return std::integral_constant<int, decltype(n)::value * ND>{}; };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+
+#pragma unroll
+  for (int st = 0; st < NBUF - 1; ++st)
+    if (st < ns) dma_stage(st, st);
+  if (NBUF >= 4 && ns > 2) wait_dma(whole(I2{}));
+  else if (ns > 1) wait_dma(whole(I1{}));
+  else wait_dma(I0{});
+  act_stage(0);
+  if (ragged && ns == 1) zero_tail(0);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  fread(0, 0, 0);
+  int cb = 0, pb_ = NBUF - 1;
+  // Iteration s: products of stage s; quarters 0..3 of stage s + NBUF - 1 (into the buffer that the
+  // previous iteration freed) go out in its four groups.
+  auto iter = [&](int s, auto dma_tag) __attribute__((always_inline)) {
+    constexpr int kDma = decltype(dma_tag)::value;
+    const int nb = cb + 1 == NBUF ? 0 : cb + 1;
+    const Src f = kDma ? src_of(pb_, s + NBUF - 1) : Src{};
+    fread(cb, 1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma(0, dma_tag, 0, f);
+    fread(cb, 2, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma(1, dma_tag, 1, f);
+    fread(cb, 3, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma(0, dma_tag, 2, f);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kDma || s + 1 < ns) {
+      // stage s + 1 has landed; in flight may be the later ones: NBUF - 3 whole stages and three
+      // quarters of the one this iteration issues, or at the end what is left
+      if constexpr (kDma != 0) wait_dma(std::integral_constant<int, (NBUF - 3) * ND + 3 * ND / 4>{});
+      else if (NBUF >= 4 && s + 2 < ns) wait_dma(whole(I1{}));
+      else wait_dma(I0{});
+      act_stage(nb);
+      if (ragged && s + 2 == ns) zero_tail(nb);
+      // this wave's reads of buffer cb have returned, every wave's stage s + 1 has landed
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      fread(nb, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    mfma(1, dma_tag, 3, f);
+    __builtin_amdgcn_sched_barrier(0);
+    pb_ = cb;
+    cb = nb;
+  };
+  int s = 0;
+  for (; s + NBUF - 1 < ns - 1; ++s) iter(s, std::integral_constant<int, 1>{});
+  if (s + NBUF - 1 < ns) {
+    if (ragged) iter(s, std::integral_constant<int, 2>{});
+    else iter(s, std::integral_constant<int, 1>{});
+    ++s;
+  }
+  for (; s < ns; ++s) iter(s, std::integral_constant<int, 0>{});
+  // every wave is done with the ring: its space stages the output
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  float* const st = reinterpret_cast<float*>(sm) + w * 32 * mid_st_row(TN);
+  const int row0 = m0 + wm * (BM / 2), col0 = n0 + wn * (BN / 2);
+  if (P.splits > 1) {
+    mid_store<TM, TN, true, VKWR_GEMM_EPI_NONE>(st, P, acc, row0, col0, split, lane);
+    return;
+  }
+  switch (P.epi) {
+    case VKWR_GEMM_EPI_RELU_SQUARE: mid_store<TM, TN, false, VKWR_GEMM_EPI_RELU_SQUARE>(st, P, acc, row0, col0, 0, lane); break;
+    case VKWR_GEMM_EPI_VALUE_RESIDUAL: mid_store<TM, TN, false, VKWR_GEMM_EPI_VALUE_RESIDUAL>(st, P, acc, row0, col0, 0, lane); break;
+    case VKWR_GEMM_EPI_BIAS: mid_store<TM, TN, false, VKWR_GEMM_EPI_BIAS>(st, P, acc, row0, col0, 0, lane); break;
+    case VKWR_GEMM_EPI_TANH: mid_store<TM, TN, false, VKWR_GEMM_EPI_TANH>(st, P, acc, row0, col0, 0, lane); break;
+    case VKWR_GEMM_EPI_SIGMOID: mid_store<TM, TN, false, VKWR_GEMM_EPI_SIGMOID>(st, P, acc, row0, col0, 0, lane); break;
+    default: mid_store<TM, TN, false, VKWR_GEMM_EPI_NONE>(st, P, acc, row0, col0, 0, lane); break;
+  }
+}
+
+// Adds the K parts of the mid-size path's split problems (blockIdx.y: the problem), 8 consecutive
+// outputs per thread, parts in increasing order with 4 of them in flight, and applies the epilogue.
+__global__ __launch_bounds__(256) void mid_reduce_kernel(Batch bt) {
+  const Prob& P = bt.p[blockIdx.y];
+  {
+    const _Float16 *fv = P.v, *fvf = P.vf, *fv0 = P.v0;
+    _Float16* fc = P.c;
+    float* fws = P.ws;
+    const int f0 = P.m, f1 = P.n, f2 = P.epi, f3 = P.splits, f4_ = P.vec_out;
+    asm volatile("" ::"s"(fv), "s"(fvf), "s"(fv0), "s"(fc), "s"(fws), "s"(f0), "s"(f1), "s"(f2), "s"(f3), "s"(f4_));
+  }
+  if (P.splits <= 1) return;
+  const int64_t mn = (int64_t)P.m * P.n;  // a multiple of 8
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < mn; i += (int64_t)gridDim.x * 256 * 8) {
+    float s8[8];
+    for (int z = 0; z < P.splits; z += 4) {
+      float v[4][8];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float* p = P.ws + (int64_t)min(z + u, P.splits - 1) * mn + i;
+        if (P.vec_out) {
+          const f4 lo = *reinterpret_cast<const f4*>(p), hi = *reinterpret_cast<const f4*>(p + 4);
+          v[u][0] = lo.x, v[u][1] = lo.y, v[u][2] = lo.z, v[u][3] = lo.w;
+          v[u][4] = hi.x, v[u][5] = hi.y, v[u][6] = hi.z, v[u][7] = hi.w;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[u][e] = p[e];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (z + u < P.splits) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) s8[e] = z + u == 0 ? v[u][e] : s8[e] + v[u][e];
+        }
+    }
+    const int row = (int)(i / P.n), col = (int)(i % P.n);
+    hv8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float y = epilogue(P, s8[e], row, col + e);
+      asm volatile("" : "+v"(y));  // round in fp32, then to fp16 (no fused mixed-precision op)
+      o[e] = (_Float16)y;
+    }
+    *reinterpret_cast<hv8*>(P.c + i) = o;
+  }
+}
+
 // ---- small-M path (decode-sized batches, M <= 128): row-major operands staged through LDS.
 //
 // At M <= 128 every weight byte is used M times, so the launch streams the weights
@@ -1461,6 +1893,7 @@ struct Config {
   bool rm = false;  // gemm_rm_kernel (bm x bn tiles, K split over its waves, no workspace)
   bool kn = false;  // ... with [K,N] weights
   int gv = 0;       // gemv_{nk,kn}_kernel<gv> (M <= gv <= 4), 0: not this path
+  int mid = 0;      // gemm_mid_kernel (bm x bn tiles, K in `mid` parts), 0: not this path
 };
 
 // Tile shape from the largest M of the batch (all problems of one launch share it).
@@ -1575,14 +2008,11 @@ bool gv_config(const Batch& bt, int max_m, Config& cfg) {
   return true;
 }
 
-int64_t plan_big(Batch& bt, BigPlan& pl);
+int64_t plan_big(Batch& bt, BigPlan& pl, double* us);
+int mid_splits(const Prob& P, int parts);
 
 // Fills tiling fields and returns the workspace bytes the batch needs.
 int64_t plan(Batch& bt, Config cfg, int target_wgs) {
-  if (cfg.big) {
-    BigPlan pl;
-    return plan_big(bt, pl);
-  }
   if (cfg.gv) {
     // [K,N]: split K over workgroups until the batch has a workgroup per CU, each part >= 128
     // k rows (a multiple of 32) whose activation slice fits the staging buffer.
@@ -1643,6 +2073,23 @@ int64_t plan(Batch& bt, Config cfg, int target_wgs) {
         P.k_per_split = P.splits > 1 ? kps : P.k;
         if (P.splits > 1) ws += (int64_t)P.splits * P.m * P.n * 4;
       }
+      P.tile_begin = begin;
+      begin += P.tiles_m * P.tiles_n * P.splits;
+    }
+    return ws;
+  }
+  if (cfg.mid) {
+    int64_t ws = 0;
+    int begin = 0;
+    for (int i = 0; i < bt.n; ++i) {
+      Prob& P = bt.p[i];
+      const bool empty = P.m == 0 || P.n == 0;
+      P.tiles_m = empty ? 0 : (P.m + cfg.bm - 1) / cfg.bm;
+      P.tiles_n = empty ? 0 : (P.n + cfg.bn - 1) / cfg.bn;
+      const int s = empty ? 1 : mid_splits(P, cfg.mid), stages = (P.k + kMidBK - 1) / kMidBK;
+      P.splits = s;
+      P.k_per_split = s > 1 ? (stages + s - 1) / s * kMidBK : P.k;
+      if (P.splits > 1) ws += (int64_t)P.splits * P.m * P.n * 4;
       P.tile_begin = begin;
       begin += P.tiles_m * P.tiles_n * P.splits;
     }
@@ -1771,11 +2218,13 @@ double plan_big_bm(Batch& bt, BigPlan& pl, int BM) {
 // Picks the tile rows (256, or 192 when its plan is estimated to be at least 5 % faster -- M =
 // 2304 fills 256 CUs with 192 row tiles far better than with 144 -- or, for unequal K, fills
 // the last round better) and plans the batch; returns the workspace bytes the plan needs.
-int64_t plan_big(Batch& bt, BigPlan& pl) {
+// (and, in *us, the plan's estimated time or negative fill).
+int64_t plan_big(Batch& bt, BigPlan& pl, double* us) {
   BigPlan p192;
   const double t192 = plan_big_bm(bt, p192, 192);
-  const double t256 = plan_big_bm(bt, pl, 256);
-  if (t256 < 0 ? t192 < t256 - 0.05 : t192 < 0.95 * t256) plan_big_bm(bt, pl, 192);
+  double t256 = plan_big_bm(bt, pl, 256);
+  if (t256 < 0 ? t192 < t256 - 0.05 : t192 < 0.95 * t256) t256 = plan_big_bm(bt, pl, 192);
+  *us = t256;
   if (pl.sk_tiles == 0) return 0;
   int64_t slots = (int64_t)pl.sk_tiles * pl.parts;
   if (pl.wgs > 0) {
@@ -1785,13 +2234,179 @@ int64_t plan_big(Batch& bt, BigPlan& pl) {
   return slots * pl.bm * kBigBM * 4;
 }
 
+// ---- choice of the mid-size path.
+//
+// K parts of problem P when the batch asks for `parts`: at least 4 stages each.
+int mid_splits(const Prob& P, int parts) {
+  const int stages = (P.k + kMidBK - 1) / kMidBK;
+  const int s = std::max(1, std::min(parts, stages / 4));
+  const int kps = (stages + s - 1) / s;
+  return (stages + kps - 1) / kps;
+}
+
+// gemm_mid_kernel takes a batch when every non-empty problem has 16-byte rows (operands and
+// output), K a multiple of 8 and >= 8, operands below 4 GiB (32-bit DMA offsets), one weight
+// layout, and some problem more than 64 rows.
+bool mid_eligible(const Batch& bt, int max_m) {
+  if (max_m <= 64) return false;
+  int kn = -1;
+  for (int i = 0; i < bt.n; ++i) {
+    const Prob& P = bt.p[i];
+    if (P.m == 0 || P.n == 0) continue;
+    if (!P.vec || !P.vec_out || P.k < 8 || (kn >= 0 && kn != P.b_kn)) return false;
+    kn = P.b_kn;
+    if ((int64_t)std::max(P.m, P.n) * P.k * 2 > 0xFFFF0000LL) return false;
+  }
+  return kn >= 0;
+}
+
+// Bytes of a batch's operands and outputs over the rate at which launches of this size stream
+// weights (3.7 TB/s measured: 2048 x 65536 at M = 128 in 74 us), plus ~5 us of ramp: no tile
+// shape goes below it.
+double gemm_stream_us(const Batch& bt) {
+  double bytes = 0;
+  for (int i = 0; i < bt.n; ++i) {
+    const Prob& P = bt.p[i];
+    if (P.m == 0 || P.n == 0) continue;
+    const int per_out = P.epi == VKWR_GEMM_EPI_VALUE_RESIDUAL ? 3 : 1;
+    bytes += 2.0 * ((double)P.n * P.k + (double)P.m * P.k + (double)per_out * P.m * P.n);
+  }
+  return 5.0 + bytes / 3.7e6;
+}
+
+// Estimated time (us) of the batch as BM x BN tiles with K in up to `parts` parts, and the
+// workspace that takes.  Fitted to sweeps over M = 64..3000 and (K, N) from (96, 2048) to
+// (16384, 4096): a workgroup costs `over` (first loads, output) plus its stages; a stage takes
+// longer the more CUs are busy (L2 and fabric).  64 x 64 tiles sit two to a CU, the others one.
+//   64 x 64    M = 512, K = N = 2048 (256 tiles)          13.9 modelled, 10.4 measured
+//   128 x 128  M = 2048, K = N = 2048 (256 tiles)         20.2, 19.6
+//   256 x 128  M = 512, K = 4096, N = 16384 (256 tiles)   66.2, 66.6
+double mid_estimate(const Batch& bt, int G, int bm, int bn, int parts, bool unequal, double floor_us, int64_t* ws,
+                    int* tiles) {
+  const bool two = bm == 64;  // two workgroups per CU
+  const int lm = bm == 64 ? 6 : bm == 128 ? 7 : 8, ln = bn == 64 ? 6 : bn == 128 ? 7 : 8;
+  int W = 0, longest = 0;     // workgroups; most stages of one
+  int64_t work = 0, mn = 0;   // stages of all; partial sums
+  double acts = 0, out = 0;   // stages of problems with an A activation; output bytes
+  for (int i = 0; i < bt.n; ++i) {
+    const Prob& P = bt.p[i];
+    if (P.m == 0 || P.n == 0) continue;
+    const int stages = (P.k + kMidBK - 1) / kMidBK, s = mid_splits(P, parts);
+    const int wgs = ((P.m + bm - 1) >> lm) * ((P.n + bn - 1) >> ln) * s;
+    W += wgs;
+    longest = std::max(longest, s > 1 ? (stages + s - 1) / s : stages);
+    work += (int64_t)wgs / s * stages;
+    if (P.a_act != VKWR_GEMM_ACT_NONE) acts += (double)wgs / s * stages;
+    if (s > 1) mn += (int64_t)s * P.m * P.n;
+    out += 2.0 * P.m * P.n;
+  }
+  *ws = mn * 4;
+  *tiles = W;
+  const int slots = two ? 2 * G : G;
+  const double fill = std::min(1.0, (double)W / G);
+  const bool sq = bm == 128 && bn == 128;
+  const double t0 = two ? 3.2 : 1.8, over = two ? (W <= slots ? 0.6 : 2.1) : (sq ? 3.0 : 4.2);
+  double stage = two ? (W <= G ? 0.20 : 0.27 + 0.14 * std::min(1.0, (double)W / slots))
+                     : (sq ? (W <= G ? 0.36 + 0.16 * fill : 0.56) : 0.60 + 0.34 * fill);
+  if (bn == 256) stage *= 1.02;
+  const double act = 0.0066 * bm;  // a stage's activations: ~64 clocks per wave and value
+  const double mean = over + (work * stage + acts * act) / W;
+  double t = over + longest * (stage + (acts > 0 ? act : 0.0));
+  if (W > slots) {
+    t = mean * ((W + slots - 1) / slots);
+    if (two && W % slots && W % slots <= G) t -= mean * 0.4;  // a last round of one per CU
+    if (!two && unequal) t += out / 5e6;                      // short K: output in the open
+  }
+  t = std::max(t0 + t, floor_us) + 0.1 * t;  // (at the floor, the shape with less to do)
+  if (mn > 0) t += 3.3 + (double)mn * 8 / 6e6;  // the reduce launch and its traffic
+  return t;
+}
+
+// Estimated time (us) of a planned large-M batch: plan_big_bm's, with a stage shorter while CUs
+// are idle (M = 400, K = 4096, N = 16384: 128 tiles in 87 us, 256 tiles at M = 1000 in 121) and,
+// for unequal K (the low-rank outputs: short K), ~10 us of output per tile (M = 2304, N = 4096, K
+// = 128..512: 768 tiles in 53 us; M = 1048: 384 in 31).
+double big_estimate(const Batch& bt, const BigPlan& pl, double planned) {
+  const int G = device_cus();
+  double t;
+  if (planned < 0) {
+    double sum = 0;
+    for (int i = 0; i < bt.n; ++i) {
+      const Prob& P = bt.p[i];
+      sum += (double)P.tiles_m * P.tiles_n * (P.k / kBigBK * (pl.bm == 192 ? 1.36 : 1.7) + 10.5);
+    }
+    t = 8.0 + sum / G;
+  } else if (pl.sk_tiles == 0 && pl.dp_tiles < G) {
+    int k = 0;
+    for (int i = 0; i < bt.n; ++i) k = std::max(k, bt.p[i].m > 0 && bt.p[i].n > 0 ? bt.p[i].k : 0);
+    const double f = pl.bm == 192 ? 0.8 : 1.0;
+    t = k / kBigBK * f * (0.8 + 0.9 * pl.dp_tiles / G) + 7.4;
+  } else {
+    t = planned + 4.0;
+  }
+  return 1.1 * std::max(t, gemm_stream_us(bt));
+}
+
+// Most partials (bytes) a mid-size plan may take: the scratch of vkwr_gemm_f16_noalloc.
+constexpr int64_t kMidMaxWs = (int64_t)32 << 20;
+
+// Moves the batch to gemm_mid_kernel where that is faster than `cfg`, the path chosen among
+// the others; `limit` bounds the workspace of its K parts.
+//  * instead of the row-major tile kernel (more than 128 rows and [K,N] weights, activations,
+//    or K no multiple of 64; or 129..255 rows): always -- K = N = 2048 at M = 200: 26.5 -> 10.0
+//    us, [K,N] at M = 1024: 122.9 -> 18, K = 8192, N = 2048 [K,N] at M = 777: 511 -> 43.
+//  * instead of the large-M kernel: where the estimates say so (M = 512, K = N = 2048: 33.2 ->
+//    10.4 us; M = 1000, K = 4096, N = 16384: 121 against 133, not taken).
+//  * instead of the small-M kernel: 65..128 rows on weights of at least 48 MiB, where that
+//    kernel's 64-row tiles fetch the weights twice -- K = 2048, N = 65536: 116 -> 75 us at M =
+//    96; at 32 MiB (4096 x 4096) the two are level (M = 128: 16.9 against 19.3).
+void mid_choose(Batch& bt, int max_m, int64_t limit, const BigPlan& pl, double planned, Config& cfg) {
+  if (cfg.gv || !mid_eligible(bt, max_m)) return;
+  double base = 1e30;
+  if (cfg.rm) {
+    int64_t weights = 0;
+    for (int i = 0; i < bt.n; ++i) weights += (int64_t)bt.p[i].n * bt.p[i].k * 2 * (bt.p[i].m > 0);
+    if (weights < (int64_t)48 << 20) return;
+  } else if (cfg.big) {
+    base = big_estimate(bt, pl, planned);
+  }
+  static const int shapes[4][2] = {{64, 64}, {128, 128}, {256, 128}, {128, 256}};
+  Config best = cfg;
+  const double floor_us = gemm_stream_us(bt);
+  const int G = device_cus();
+  bool unequal = false;
+  for (int i = 0, k = -1; i < bt.n; ++i) {
+    if (bt.p[i].m == 0 || bt.p[i].n == 0) continue;
+    unequal = unequal || (k >= 0 && bt.p[i].k != k);
+    k = bt.p[i].k;
+    best.kn = bt.p[i].b_kn != 0;
+  }
+  if (unequal && cfg.big) base *= 0.85;  // short K: level within the estimates' error from M ~ 700 up
+  for (const auto& sh : shapes)
+    for (int parts : {1, 2, 3, 4, 6, 8}) {
+      int64_t ws;
+      int wgs;
+      const double t = mid_estimate(bt, G, sh[0], sh[1], parts, unequal, floor_us, &ws, &wgs);
+      if (parts > 1 && ws == 0) break;  // K too short to split
+      if (ws <= limit && t < base) {
+        base = t;
+        best = Config{sh[0], sh[1], false, false, best.kn, 0, parts};
+      }
+      if (wgs >= G) break;  // the CUs are full: more parts only add partial sums
+    }
+  if (!best.mid) return;
+  cfg = best;
+  bt.xbal = unequal ? 1 : 0;
+  if (unequal) std::stable_sort(bt.p, bt.p + bt.n, [](const Prob& a, const Prob& b) { return a.k > b.k; });
+}
+
 int total_wgs(const Batch& bt) {
   int t = 0;
   for (int i = 0; i < bt.n; ++i) t += bt.p[i].tiles_m * bt.p[i].tiles_n * bt.p[i].splits;
   return t;
 }
 
-int build_batch(const char* fn, int n, const vkwr_gemm_problem* pr, Batch& bt, Config& cfg) {
+int build_batch(const char* fn, int n, const vkwr_gemm_problem* pr, Batch& bt, Config& cfg, int& rows) {
   VK_REQUIRE(n >= 1 && n <= kMaxProblems, "%s: 1..%d problems per launch (got %d)", fn, kMaxProblems, n);
   VK_REQUIRE(pr != nullptr, "%s: null problem list", fn);
   bt.n = n;
@@ -1836,6 +2451,7 @@ int build_batch(const char* fn, int n, const vkwr_gemm_problem* pr, Batch& bt, C
       min_n = std::min(min_n, P.n);
     }
   }
+  rows = max_m;
   cfg = pick_config(max_m, min_n);
   if (big_eligible(bt, max_m)) cfg = Config{kBigBM, kBigBM, true};
   else if (!gv_config(bt, max_m, cfg)) rm_config(bt, max_m, cfg);
@@ -1843,6 +2459,20 @@ int build_batch(const char* fn, int n, const vkwr_gemm_problem* pr, Batch& bt, C
 }
 
 constexpr int kTargetWgs = 512;  // two workgroups per CU on 256 CUs
+
+// Plans the batch with at most `limit` bytes for the mid-size path's K parts.  *need: the
+// workspace to ask for -- the plan's, and never less than the plan of the other paths takes, so
+// that what a workspace (or the fixed scratch) was too small for stays refused.
+int plan_batch(const char* fn, int n, const vkwr_gemm_problem* pr, int64_t limit, Batch& bt, Config& cfg, BigPlan& pl,
+               int64_t* need) {
+  int rows = 0;
+  double planned = 0;
+  if (int e = build_batch(fn, n, pr, bt, cfg, rows)) return e;
+  *need = cfg.big ? plan_big(bt, pl, &planned) : plan(bt, cfg, kTargetWgs);
+  mid_choose(bt, rows, std::min(limit, kMidMaxWs), pl, planned, cfg);
+  if (cfg.mid) *need = std::max(*need, plan(bt, cfg, kTargetWgs));
+  return VKWR_OK;
+}
 
 }  // namespace
 }  // namespace vk
@@ -1853,8 +2483,28 @@ extern "C" int64_t vkwr_gemm_f16_workspace_bytes(int n_problems, const vkwr_gemm
   clear_error();
   Batch bt;
   Config cfg;
-  if (build_batch("vkwr_gemm_f16_workspace_bytes", n_problems, problems, bt, cfg)) return -1;
-  return plan(bt, cfg, kTargetWgs);
+  BigPlan pl;
+  int64_t need;
+  if (plan_batch("vkwr_gemm_f16_workspace_bytes", n_problems, problems, kMidMaxWs, bt, cfg, pl, &need)) return -1;
+  return need;
+}
+
+extern "C" int64_t vkwr_gemm_f16_workspace_bytes_upto(int n_problems, const vkwr_gemm_problem* problems) {
+  clear_error();
+  const char* fn = "vkwr_gemm_f16_workspace_bytes_upto";
+  Batch bt;
+  Config cfg;
+  BigPlan pl;
+  int64_t need, most = 0;
+  if (plan_batch(fn, n_problems, problems, kMidMaxWs, bt, cfg, pl, &need)) return -1;
+  vkwr_gemm_problem p[kMaxProblems];
+  std::copy(problems, problems + n_problems, p);
+  for (int64_t m = 1; m <= problems[0].m; ++m) {
+    for (int i = 0; i < n_problems; ++i) p[i].m = m;
+    if (plan_batch(fn, n_problems, p, kMidMaxWs, bt, cfg, pl, &need)) return -1;
+    most = std::max(most, need);
+  }
+  return most;
 }
 
 // Scratch of vkwr_gemm_f16_noalloc: the K-split / stream-K partials of one launch.  Each
@@ -1866,9 +2516,28 @@ static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
 
+template <int BM, int BN, int NBUF>
+void mid_launch_tile(bool kn, bool act, const Batch& bt, int wgs, hipStream_t s) {
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(wgs), dim3(256), 0, s, bt, wgs); };
+  if (kn) {
+    if (act) go(gemm_mid_kernel<BM, BN, NBUF, true, true>);
+    else go(gemm_mid_kernel<BM, BN, NBUF, true, false>);
+  } else {
+    if (act) go(gemm_mid_kernel<BM, BN, NBUF, false, true>);
+    else go(gemm_mid_kernel<BM, BN, NBUF, false, false>);
+  }
+}
+
+void mid_launch(const Config& cfg, bool act, const Batch& bt, int wgs, hipStream_t s) {
+  if (cfg.bm == 64) mid_launch_tile<64, 64, 4>(cfg.kn, act, bt, wgs, s);
+  else if (cfg.bn == 256) mid_launch_tile<128, 256, 3>(cfg.kn, act, bt, wgs, s);
+  else if (cfg.bm == 256) mid_launch_tile<256, 128, 3>(cfg.kn, act, bt, wgs, s);
+  else mid_launch_tile<128, 128, 4>(cfg.kn, act, bt, wgs, s);
+}
+
 // Launches a planned batch whose workspace (need bytes, checked by the caller) is at
 // `workspace`.  Shared by vkwr_gemm_f16 and vkwr_gemm_f16_noalloc.
-int gemm_run(const char* fn, Batch& bt, const Config& cfg, void* workspace, void* stream) {
+int gemm_run(const char* fn, Batch& bt, const Config& cfg, BigPlan& pl, void* workspace, void* stream) {
   // Zero-sized problems and K == 0: nothing to tile; K == 0 writes epilogue(0).
   float* ws = reinterpret_cast<float*>(workspace);
   for (int i = 0; i < bt.n; ++i) {
@@ -1947,9 +2616,24 @@ int gemm_run(const char* fn, Batch& bt, const Config& cfg, void* workspace, void
     }
     return VKWR_OK;
   }
+  if (cfg.mid) {
+    bool any_act = false;
+    int64_t mn = 0;  // outputs of the largest split problem
+    for (int i = 0; i < bt.n; ++i) {
+      if (bt.p[i].m == 0 || bt.p[i].n == 0) continue;
+      any_act = any_act || bt.p[i].a_act != VKWR_GEMM_ACT_NONE;
+      if (bt.p[i].splits > 1) mn = std::max(mn, (int64_t)bt.p[i].m * bt.p[i].n);
+    }
+    mid_launch(cfg, any_act, bt, wgs, s);
+    if (int e = check_launch(fn)) return e;
+    if (any_split) {
+      const int rw = (int)std::min<int64_t>(2048, (mn / 8 + 255) / 256);
+      hipLaunchKernelGGL(mid_reduce_kernel, dim3(rw, bt.n), dim3(256), 0, s, bt);
+      if (int e = check_launch(fn)) return e;
+    }
+    return VKWR_OK;
+  }
   if (cfg.big) {
-    BigPlan pl;
-    plan_big(bt, pl);  // same plan as above (need)
     pl.ws = reinterpret_cast<float*>(workspace);
     int epi = -2;  // the batch's common epilogue, -1 if they differ
     for (int i = 0; i < bt.n; ++i) {
@@ -2027,12 +2711,15 @@ extern "C" int vkwr_gemm_f16(int n_problems, const vkwr_gemm_problem* problems, 
   const char* fn = "vkwr_gemm_f16";
   Batch bt;
   Config cfg;
-  if (int e = build_batch(fn, n_problems, problems, bt, cfg)) return e;
-  const int64_t need = plan(bt, cfg, kTargetWgs);
+  BigPlan pl;
+  int64_t need;
+  // (a workspace that holds the other paths' partials but not the mid-size path's best plan
+  // bounds that plan's K parts)
+  if (int e = plan_batch(fn, n_problems, problems, workspace ? workspace_bytes : 0, bt, cfg, pl, &need)) return e;
   VK_REQUIRE(need <= workspace_bytes && (need == 0 || workspace != nullptr),
              "%s: workspace of %lld bytes needed (got %lld)", fn, (long long)need,
              (long long)workspace_bytes);
-  return gemm_run(fn, bt, cfg, workspace, stream);
+  return gemm_run(fn, bt, cfg, pl, workspace, stream);
 }
 
 extern "C" int64_t vkwr_gemm_f16_noalloc_max_bytes(void) { return kNoAllocScratchBytes; }
@@ -2046,11 +2733,12 @@ extern "C" int vkwr_gemm_f16_noalloc(int n_problems, const vkwr_gemm_problem* pr
   if (int e = scratch_ptr(fn, &ws)) return e;
   Batch bt;
   Config cfg;
-  if (int e = build_batch(fn, n_problems, problems, bt, cfg)) return e;
-  const int64_t need = plan(bt, cfg, kTargetWgs);
+  BigPlan pl;
+  int64_t need;
+  if (int e = plan_batch(fn, n_problems, problems, kNoAllocScratchBytes, bt, cfg, pl, &need)) return e;
   VK_REQUIRE(need <= kNoAllocScratchBytes,
              "%s: this batch needs %lld bytes of scratch; the allocation-free entry point holds at most "
              "%lld (use vkwr_gemm_f16 with a workspace)",
              fn, (long long)need, (long long)kNoAllocScratchBytes);
-  return gemm_run(fn, bt, cfg, need > 0 ? ws : nullptr, stream);
+  return gemm_run(fn, bt, cfg, pl, need > 0 ? ws : nullptr, stream);
 }
