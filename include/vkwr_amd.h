@@ -73,6 +73,22 @@ VKWR_EXPORT int vkwr_wkv7_fp32_forward_slots(int B, int T, int C, int H, float* 
                                  const uint16_t* a, const uint16_t* b, uint16_t* y,
                                  void* stream);
 
+/* vkwr_wkv7_fp32_forward (mode 0; slots = NULL: state is dense, [B,H,64,64]) or
+ * vkwr_wkv7_fp32_forward_slots (slots given: state is the pool) with device scratch: where
+ * the batch has too few (sequence, head) chains to fill the GPU, a long prefill is cut into
+ * segments along T that run side by side and are joined through the scratch.  Same values to
+ * fp32 rounding.  workspace: vkwr_wkv7_fp32_prefill_workspace_bytes(B, T, H) bytes, 16-byte
+ * aligned; with less, or NULL, the call runs without segments, as the entry points above.
+ * ..._workspace_max(rows, H): enough for every B, T with B * T <= rows.
+ * Replaces the device work of vkwr_v1_wkv::wkv_forward_fp32 (csrc/v1/wkv/torch_bindings.cpp:179-188). */
+VKWR_EXPORT int64_t vkwr_wkv7_fp32_prefill_workspace_bytes(int B, int T, int H);
+VKWR_EXPORT int64_t vkwr_wkv7_fp32_prefill_workspace_max(int64_t rows, int H);
+VKWR_EXPORT int vkwr_wkv7_fp32_prefill(int B, int T, int C, int H, float* state, int n_slots,
+                                       const int32_t* slots, const uint16_t* r, const uint16_t* w,
+                                       const uint16_t* k, const uint16_t* v, const uint16_t* a,
+                                       const uint16_t* b, uint16_t* y, void* workspace,
+                                       int64_t workspace_bytes, void* stream);
+
 /* One decode step (T = 1) of vkwr_wkv7_fp32_forward_slots with the dot products in the
  * row-split order of the prefill kernels (eight 8-term FMA chains per state row, combined
  * pairwise) instead of one 64-term chain, and no LDS: it can run on a second stream beside

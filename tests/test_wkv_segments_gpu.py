@@ -1,0 +1,126 @@
+"""A prefill of few (sequence, head) chains cut into segments along T: against the reference-order
+oracle at the chunked kernel's contract, over ragged lengths, slots, dense states, scratch limits
+and several blocks."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from tests.test_wkv_gpu import BIG_Y, CHUNK_Y_MEAN_REL, Y_MAX_ABS, _check_state_chunked, _dev
+from tests.wkv_inputs import make_state, make_wkv_inputs
+from vkwr_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _slow(ins, seed):
+    """The inputs with w from long to short memory across the channels (decays up to 0.998)."""
+    w = ins[1]
+    base = -6.0 + 5.0 * np.random.default_rng(seed).random(w.shape[-1])
+    ins[1] = (base + 0.5 * np.random.default_rng(seed + 1).standard_normal(w.shape)).astype(np.float16)
+    return ins
+
+
+def _one_chain(B, T, H, state_np, ins, gpu):
+    """y of the form without segments (no scratch)."""
+    y = torch.empty(B, T, H * 64, dtype=torch.float16, device=gpu)
+    capi.wkv_slots(B, T, H * 64, H, torch.from_numpy(state_np.copy()).to(gpu),
+                   torch.arange(B, dtype=torch.int32, device=gpu), *_dev(ins, gpu), y)
+    torch.cuda.synchronize()
+    return y
+
+
+def _check_y(y, plain, y_ref, what):
+    """_check_y_chunked's bounds but for its share of differing values, which it states for short
+    memory: with decays up to 0.998 every fp32 form's error is larger against the fp16 spacing, so
+    the share is held to twice that of the one-chain form on the same inputs (the segmented
+    form's error against 64 bits is 1.25 times the one-chain form's)."""
+    yr = y_ref.astype(np.float64)
+    yg, yp = (t.cpu().numpy().astype(np.float64) for t in (y, plain))
+    err = np.abs(yg - yr)
+    ulp = np.exp2(np.floor(np.log2(np.maximum(np.abs(yr), 2.0 ** -14))) - 10)
+    big = np.abs(yr) >= BIG_Y
+    assert (err[big] <= ulp[big]).all() and (err[~big] <= Y_MAX_ABS).all(), (what, float(err.max()))
+    assert err.sum() <= CHUNK_Y_MEAN_REL * np.abs(yr).sum(), (what, err.sum() / np.abs(yr).sum())
+    assert (yg != yr).sum() <= 2 * (yp != yr).sum() + 10, (what, (yg != yr).sum(), (yp != yr).sum())
+
+
+@pytest.mark.parametrize("B,T,H,memory", [
+    (1, 512, 2, "short"),   # whole chunks
+    (1, 337, 12, "long"),   # a last chunk of one token
+    (2, 1023, 3, "long"),   # two sequences, a last chunk one token short
+    (1, 1500, 32, "short"),
+    (3, 700, 20, "long"),   # segments that do not divide the chunks
+    (1, 4096, 1, "long"),   # as many segments as the model takes
+])
+def test_segments_match_oracle(gpu, B, T, H, memory):
+    from vkwr._ops.v1 import v1_wkv_ops as ops
+
+    C, P = H * 64, 2 * B + 3
+    pool_np = make_state(P, H, seed=T)
+    slots_np = np.random.default_rng(T).permutation(P)[:B].astype(np.int32)
+    ins = make_wkv_inputs(B, T, H, seed=T, dist="realistic")
+    if memory == "long":
+        ins = _slow(ins, T)
+    assert capi._LIB.vkwr_wkv7_fp32_prefill_workspace_bytes(B, T, H) > 0  # the segmented form runs
+    pool = torch.from_numpy(pool_np.copy()).to(gpu)
+    dense = pool[slots_np.tolist()].clone()
+    y = ops.wkv_forward_slots_fp32(B, T, C, H, pool, torch.from_numpy(slots_np).to(gpu), *_dev(ins, gpu))
+    yd = ops.wkv_forward_fp32(B, T, C, H, dense, *_dev(ins, gpu))
+    plain = _one_chain(B, T, H, pool_np[slots_np], ins, gpu)
+    y_ref = orc.wkv_fp32_slots(B, T, C, H, pool_np, slots_np.astype(np.int64), *ins, order="seq")
+    _check_y(y, plain, y_ref, (B, T, H))
+    _check_state_chunked(pool[slots_np.tolist()], pool_np[slots_np], (B, T, H))
+    others = np.setdiff1d(np.arange(P), slots_np)
+    assert np.array_equal(pool[others.tolist()].cpu().numpy(), pool_np[others])
+    assert torch.equal(y, yd) and torch.equal(dense, pool[slots_np.tolist()])
+
+
+def test_segments_over_several_blocks(gpu):
+    """More tokens than one block's scratch holds: the state carries from block to block."""
+    from vkwr._ops.v1 import v1_wkv_ops as ops
+
+    B, T, H = 1, 100003, 2
+    need = capi._LIB.vkwr_wkv7_fp32_prefill_workspace_bytes(B, T, H)
+    assert 0 < need < 2 * T * H * 64 * 4  # not all of T at once
+    ins = _slow(make_wkv_inputs(B, T, H, seed=5, dist="realistic"), 5)
+    S = make_state(B, H, seed=5)
+    state = torch.from_numpy(S.copy()).to(gpu)
+    y = ops.wkv_forward_fp32(B, T, H * 64, H, state, *_dev(ins, gpu))
+    plain = _one_chain(B, T, H, S, ins, gpu)
+    y_ref = orc.wkv_fp32(B, T, H * 64, H, S, *ins)
+    _check_y(y, plain, y_ref, "blocks")
+    _check_state_chunked(state, S, "blocks")
+
+
+def test_segments_out_of_range_slot_and_short_scratch(gpu):
+    """An out-of-range slot: NaN rows, every other sequence and slot as without it.  With too little
+    scratch, none, or one that is not 16-byte aligned the call runs one chain per workgroup."""
+    B, T, H = 2, 400, 4
+    C = H * 64
+    ins = _dev(_slow(make_wkv_inputs(B, T, H, seed=9, dist="realistic"), 9), gpu)
+    pool0 = torch.from_numpy(make_state(5, H, seed=9)).to(gpu)
+    need = capi._LIB.vkwr_wkv7_fp32_prefill_workspace_bytes(B, T, H)
+    assert 0 < need <= capi.wkv_prefill_workspace_max(B * T, H)
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=gpu)
+
+    def run(slots, workspace):
+        pool, y = pool0.clone(), torch.zeros(B, T, C, dtype=torch.float16, device=gpu)
+        capi.wkv_slots(B, T, C, H, pool, torch.tensor(slots, dtype=torch.int32, device=gpu), *ins, y,
+                       workspace=workspace)
+        torch.cuda.synchronize()
+        return y, pool
+
+    y, pool = run([3, 1], ws[:need])
+    yb, poolb = run([3, 7], ws[:need])
+    assert torch.isnan(yb[1]).all() and torch.equal(yb[0], y[0])
+    assert torch.equal(poolb[3], pool[3]) and torch.equal(poolb[[0, 1, 2, 4]], pool0[[0, 1, 2, 4]])
+    plain, plain_pool = run([3, 1], None)
+    for workspace in (ws[:need - 1], ws[1:need + 1], torch.empty(0, dtype=torch.uint8, device=gpu)):
+        got, got_pool = run([3, 1], workspace)
+        assert torch.equal(got, plain) and torch.equal(got_pool, plain_pool)
+    # the two forms differ by fp32 rounding (the state contract's 2e-5 of the largest value bounds
+    # what a y that cancels can see of it), then by at most one fp16 ulp of y
+    err = (y.float() - plain.float()).abs()
+    ulp = torch.exp2(torch.floor(torch.log2(plain.float().abs().clamp_min(2.0 ** -14))) - 10)
+    assert bool((err <= ulp + 2e-5 * plain.float().abs().max()).all()) and (pool - plain_pool).abs().max().item() <= 2e-5 * plain_pool.abs().max().item()

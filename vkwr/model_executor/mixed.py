@@ -98,6 +98,8 @@ class MixedEngine:
         need = max(capi.gemm_workspace_bytes_upto(ps) for ps in self._gemm_batches(max_rows, 1))
         need = max(need, capi.gemm_workspace_bytes_upto(self._head_problem(self.max_seqs)))
         self.ws = torch.empty(max(need, 0), dtype=torch.uint8, device=dev)
+        # Scratch of the prefill chunks' WKV (segments of few long chains), used on the step's stream.
+        self.wkv_ws = torch.empty(capi.wkv_prefill_workspace_max(max_rows, cfg.n_head), dtype=torch.uint8, device=dev)
         # The decode rows' WKV step runs on a second stream beside the prefill chunks' (its
         # kernel uses no LDS, so it fits on the CUs the chunk kernel holds); default priority.
         self.side = torch.cuda.Stream(device=dev) if dev.type == "cuda" else None
@@ -164,7 +166,7 @@ class MixedEngine:
             s.fork.record(main)
         for B, T, r0, slots, _ in groups:
             if T > 1:
-                capi.wkv_slots(B, T, C, H, pool, slots, *args(r0, B * T))
+                capi.wkv_slots(B, T, C, H, pool, slots, *args(r0, B * T), workspace=s.wkv_ws)
                 gn(r0, B * T)
         for B, _, r0, slots, _ in dec:
             s.side.wait_event(s.fork)

@@ -78,6 +78,10 @@ _gate = _sig("vkwr_tmix_kk_a_gate_f16", [_i, _i, _i, _i, _p, _p, _p, _p, _p, _p,
 _gn = _sig("vkwr_tmix_groupnorm_bonus_gate_f16", [_i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p])
 _wkv_slots = _sig("vkwr_wkv7_fp32_forward_slots",
                   [_i, _i, _i, _i, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p])
+_wkv_prefill = _sig("vkwr_wkv7_fp32_prefill",
+                    [_i, _i, _i, _i, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p])
+_wkv_prefill_ws = _sig("vkwr_wkv7_fp32_prefill_workspace_bytes", [_i, _i, _i], _i64)
+_wkv_prefill_max = _sig("vkwr_wkv7_fp32_prefill_workspace_max", [_i64, _i], _i64)
 _wkv_step_rows = _sig("vkwr_wkv7_fp32_step_rows_slots", [_i, _i, _i, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p])
 _frag_gemm = _sig("vkwr_frag_gemm_f16", [_i, ctypes.POINTER(FragProblem), _p])
 _act = _sig("vkwr_activation_f16", [_i, _i64, _p, _p, _p])
@@ -301,7 +305,19 @@ def _arr_frag(problems):
     return (FragProblem * len(problems))(*problems)
 
 
-def wkv_slots(B, T, C, H, pool, slots, r, w, k, v, a, b, y):
+def wkv_prefill_workspace_max(rows, H):
+    """Bytes of scratch that wkv_slots can use for any B sequences of T tokens with B T <= rows."""
+    return _wkv_prefill_max(rows, H)
+
+
+def wkv_slots(B, T, C, H, pool, slots, r, w, k, v, a, b, y, workspace=None):
+    """WKV-7 on a slot pool; workspace: a uint8 device tensor for the segments of a long prefill of
+    few sequences (vkwr_wkv7_fp32_prefill), which runs as one chain each without it."""
+    if workspace is not None:
+        _check(_wkv_prefill(B, T, C, H, _ptr(pool), pool.shape[0], _idx(slots, B, "slots"), _ptr(r), _ptr(w), _ptr(k),
+                            _ptr(v), _ptr(a), _ptr(b), _ptr(y), _ptr(workspace), workspace.numel(), _stream()),
+               "vkwr_wkv7_fp32_prefill")
+        return
     _check(_wkv_slots(B, T, C, H, _ptr(pool), pool.shape[0], _idx(slots, B, "slots"), _ptr(r), _ptr(w), _ptr(k),
                       _ptr(v),
                       _ptr(a), _ptr(b), _ptr(y), _stream()), "vkwr_wkv7_fp32_forward_slots")

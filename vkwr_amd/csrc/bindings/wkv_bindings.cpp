@@ -135,6 +135,19 @@ void check_wkv_fp32_io(int64_t B, int64_t T, int64_t C, int64_t H, const at::Ten
   check_fits_int(C, "C");
 }
 
+// Mode 0 / slot pool with the scratch of a segmented prefill from torch's caching allocator.
+int wkv_prefill(int64_t B, int64_t T, int64_t C, int64_t H, at::Tensor& state, int64_t n_slots, const int32_t* slots,
+                const at::Tensor& r, const at::Tensor& w, const at::Tensor& k, const at::Tensor& v,
+                const at::Tensor& a, const at::Tensor& b, at::Tensor& y) {
+  const int64_t bytes = vkwr_wkv7_fp32_prefill_workspace_bytes((int)B, (int)T, (int)H);
+  at::Tensor ws;
+  if (bytes > 0) ws = at::empty({bytes}, r.options().dtype(at::kByte));
+  return vkwr_wkv7_fp32_prefill((int)B, (int)T, (int)C, (int)H, ptr<float>(state), (int)n_slots, slots,
+                                ptr<uint16_t>(r), ptr<uint16_t>(w), ptr<uint16_t>(k), ptr<uint16_t>(v),
+                                ptr<uint16_t>(a), ptr<uint16_t>(b), ptr<uint16_t>(y),
+                                bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream());
+}
+
 void wkv_fp32_mode(int64_t B, int64_t T, int64_t C, int64_t H, at::Tensor& state,
                    const at::Tensor& r, const at::Tensor& w, const at::Tensor& k,
                    const at::Tensor& v, const at::Tensor& a, const at::Tensor& b, at::Tensor& y,
@@ -148,6 +161,10 @@ void wkv_fp32_mode(int64_t B, int64_t T, int64_t C, int64_t H, at::Tensor& state
                   state.size(3) == 64,
               "state must have shape [B,H,64,64]");
   check_device(state, "state");
+  if (mode == 0) {
+    check_status(wkv_prefill(B, T, C, H, state, B, nullptr, r, w, k, v, a, b, y), what);
+    return;
+  }
   const int st = vkwr_wkv7_fp32_forward(
       (int)B, (int)T, (int)C, (int)H, mode, ptr<float>(state), ptr<uint16_t>(r), ptr<uint16_t>(w),
       ptr<uint16_t>(k), ptr<uint16_t>(v), ptr<uint16_t>(a), ptr<uint16_t>(b), ptr<uint16_t>(y),
@@ -195,10 +212,7 @@ void wkv_forward_slots_fp32(int64_t B, int64_t T, int64_t C, int64_t H, at::Tens
   check_wkv_fp32_io(B, T, C, H, r, w, k, v, a, b, y);
   check_fits_int(state_pool.size(0), "pool size");
   check_device(state_pool, "state_pool");
-  const int st = vkwr_wkv7_fp32_forward_slots(
-      (int)B, (int)T, (int)C, (int)H, ptr<float>(state_pool), (int)state_pool.size(0),
-      ptr<int32_t>(slots), ptr<uint16_t>(r), ptr<uint16_t>(w), ptr<uint16_t>(k), ptr<uint16_t>(v),
-      ptr<uint16_t>(a), ptr<uint16_t>(b), ptr<uint16_t>(y), stream());
+  const int st = wkv_prefill(B, T, C, H, state_pool, state_pool.size(0), ptr<int32_t>(slots), r, w, k, v, a, b, y);
   check_status(st, "wkv_forward_slots_fp32");
 }
 

@@ -770,7 +770,7 @@ __global__ __launch_bounds__(256) void wkv7_fp32_rows_kernel(RowsArgs ra) {
 // Pipeline (one barrier per chunk): in iteration c the state waves run chunk c against the
 // state (Â X0^T, R̂ X0^T, K̂^T V, then Z = W RHS, Y and B̂^T Z: the dependent chain of a
 // chunk), while matrix waves 4-7 prepare chunk c + 3's hat vectors (VALU work: Λ by a
-// multiplicative DPP scan over the 16 lanes that hold one channel quad's tokens), chunk
+// DPP scan of the log decays over the 16 lanes that hold one channel quad's tokens), chunk
 // c + 2's four L x L matrices and chunk c + 1's W^T from its N (described at the kernel).
 // Per chunk: 80 MFMAs on each state wave, 116 / 112 / 96 / 96 on the four SIMDs.  Measured
 // at config 2: 0.174 ms per call (0.24 ms for the form with four waves, each running all
@@ -796,19 +796,19 @@ __device__ __forceinline__ fq4 mfma4(float a, float b, fq4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// exp(-e^{-1/2} sigmoid(w)) from the hardware exp2 / reciprocal (about 2 ulp): the chunked
-// form is not bit-matched to the token-by-token kernels anyway, and decay() with expf's
-// range checks and an IEEE division is several times longer
-__device__ __forceinline__ float decay_fast(float w) {
+// log2 of the decay exp(-e^{-1/2} sigmoid(w)), from the hardware exp2 / reciprocal: the chunked form
+// is not bit-matched to the token-by-token kernels anyway, and decay() with expf's range checks
+// and an IEEE division is several times longer
+__device__ __forceinline__ float log2_decay_fast(float w) {
   const float e = __builtin_amdgcn_exp2f(w * -1.4426950408889634f);  // exp(-w)
-  return __builtin_amdgcn_exp2f(-0.8750387749145276f * __builtin_amdgcn_rcpf(1.0f + e));  // e^{-1/2} log2(e)
+  return -0.8750387749145276f * __builtin_amdgcn_rcpf(1.0f + e);     // e^{-1/2} log2(e)
 }
 
 typedef const __attribute__((address_space(1))) hv8 global_hv8;
 
-// x * (the value of the lane `n` below in the same 16-lane row, 1 for the first n lanes)
-#define VK_SCAN_MUL(x, ctrl) \
-  x *= __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, 1.0f), __builtin_bit_cast(int, x), ctrl, 0xF, 0xF, false))
+// x + (the value of the lane `n` below in the same 16-lane row, 0 for the first n lanes)
+#define VK_SCAN_ADD(x, ctrl) \
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), ctrl, 0xF, 0xF, false))
 
 struct ChunkLds {
   // fp16 r, w, k, v, a, b: [vec][t][8 x 8 channels + 8 of padding].  The padding spreads the
@@ -824,6 +824,31 @@ struct ChunkLds {
   __attribute__((aligned(16))) float lamSink[256];           // Λ stores of lanes that hold no Λ_L
 };
 
+// ---- a prefill of few (sequence, head) chains, cut into segments along T.
+//
+// One workgroup per chain leaves most CUs idle while its chunks run one after the other (one
+// prompt of the 1.5B shape: 32 of 256 CUs, 2.35 us a chunk).  The recurrence is linear in the
+// state: over a segment, S_end = S_start M + N with M the product of its transitions and N the
+// state it reaches from zero, and y_t = S_start q_t + y0_t with q_t = M_{<=t} r_t.  So the chain is
+// cut into P segments of cps chunks that run side by side:
+//   1. wkv7_fp32_chunk_kernel<.., kSeg>: M, N, and q_t, y0_t of every token (136 products per chunk
+//      on a state wave instead of 80);
+//   2. wkv_seg_chain_kernel: per chain, S_start of each segment in turn (P - 1 products of 64 x 64
+//      matrices) and the final state;
+//   3. wkv_seg_out_kernel: y = y0 + S_start q, all tokens at once.
+// Everything between the launches is fp32.  The products of step 2 and 3 only re-associate the
+// sums of the one-chain form: against 64 bits the state is off by 3.4e-7 (one chain 2.7e-7; 3.8e-7
+// with Λ formed as a product), y by its fp16 rounding.  T is taken in blocks of `len` tokens so
+// that the scratch stays bounded.  What bounds it: 3.4 us per chunk of a segment (the state waves'
+// products) and ~26 us of pipeline fill and launches; 32 chains, T = 1500: 220 -> 75 us.
+struct SegArgs {
+  int P, cps;    // segments, chunks per segment
+  int t0, len;   // tokens of this block
+  float *m, *n;  // [chains][P][64][64]
+  float* start;  // [chains][P][64][64] S_start of every segment
+  float *q, *y0; // [B][len][C]
+};
+
 // Eight waves in two roles, two per SIMD (waves w and w + 4 share SIMD w), so that each
 // SIMD interleaves two independent instruction streams.  State waves 0-3 own the state rows
 // and run chunk c's state products.  Matrix waves 4-7 prepare the chunks ahead of it: all four
@@ -833,18 +858,28 @@ struct ChunkLds {
 // products off the iteration that produces N and balances the matrix work over the SIMDs
 // (116 / 112 / 96 / 96 products per SIMD and chunk).  One barrier per chunk.  The LDS
 // pipeline (four hat buffers, three matrix buffers) takes 144 KiB: one workgroup per CU.
-template <bool kSlots>
-__global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra) {
+//
+// kSeg: the first of the three launches of a prefill cut into segments (SegArgs below).  The
+// workgroup takes one segment of the (sequence, head) from an unknown start state: its state
+// waves run the same chunk products on two states, M from the identity without the v k^T
+// updates, and N from zero, and store for every token M's output (the query that the start
+// state will meet) and N's, in fp32, and at the end M and N.
+template <bool kSlots, bool kSeg>
+__global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra, SegArgs sg) {
   const Fp32Args& p = ra.a;
   __shared__ ChunkLds L;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 15, g = lane >> 4;
   const bool state_wave = w < 4;
   const int mtid = tid & 255;  // thread index inside its role
-  const int bh = blockIdx.x, bi = bh / p.H, h = bh - bi * p.H;
-  const int T = p.T, C = p.C;
-  const size_t tok0 = (size_t)bi * T * C + (size_t)h * kHead;
+  const int bh = kSeg ? blockIdx.x / sg.P : blockIdx.x, bi = bh / p.H, h = bh - bi * p.H;
+  const int C = p.C;
+  // tokens of this workgroup: all, or segment seg of the block [t0, t0 + len)
+  const int seg = kSeg ? blockIdx.x - bh * sg.P : 0, s0 = seg * sg.cps * kCL;
+  const int T = kSeg ? min(sg.len - s0, sg.cps * kCL) : p.T;
+  const size_t tok0 = ((size_t)bi * p.T + (kSeg ? sg.t0 + s0 : 0)) * C + (size_t)h * kHead;
   float* S = state_block<kSlots>(p, bi, h);
+  if (kSeg && S == nullptr) return;  // the last launch writes its rows
   if (S == nullptr) {
     for (int idx = tid; idx < T * kHead; idx += 512)
       p.y[tok0 + (size_t)(idx / kHead) * C + (idx % kHead)] = (_Float16)__builtin_nanf("");
@@ -853,7 +888,17 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra) {
   const int iw = 16 * (w & 3) + li;  // a state wave lane's state row (value index), accumulator layout
   // X^T tile q (j = 16 q .. 16 q + 15): register r holds X^T[16 q + 4 g + r][iw] = S[iw][16 q + 4 g + r]
   fq4 st[4];
-  if (state_wave) {
+  fq4 sm[4];  // (kSeg) the same of M; st is N
+  if (kSeg) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        st[q][r] = 0.0f;
+        sm[q][r] = 16 * q + 4 * g + r == iw ? 1.0f : 0.0f;
+      }
+  }
+  if (!kSeg && state_wave) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) st[q] = *reinterpret_cast<const fq4*>(S + iw * kHead + 16 * q + 4 * g);
     // the loads are waited for here: otherwise the loop keeps their waits, which in every
@@ -909,26 +954,29 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra) {
     const int b = cc & 3;
     const int n = min(kCL, T - cc * kCL);
     const float in = ht < n ? 1.0f : 0.0f;  // padded tokens: d = 1 and zero vectors (a select, no branch)
-    float l1[4], l0[4];
+    float l1[4], l0[4], rl[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      float d = __builtin_fmaf(in, decay_fast((float)x.w[e]), 1.0f - in);
-      VK_SCAN_MUL(d, 0x111);  // row_shr:1
-      VK_SCAN_MUL(d, 0x112);  // row_shr:2
-      VK_SCAN_MUL(d, 0x114);  // row_shr:4
-      VK_SCAN_MUL(d, 0x118);  // row_shr:8
-      l1[e] = d;              // Λ_t
+      // Λ_t = 2^(sum of the log decays): one rounding of an exp2 per token of the chunk instead of
+      // the product's one per factor (state off 64 bits by 2.7e-7 instead of 3.8e-7 over 1500 tokens), at the
+      // same number of instructions
+      float d = in * log2_decay_fast((float)x.w[e]);
+      VK_SCAN_ADD(d, 0x111);  // row_shr:1
+      VK_SCAN_ADD(d, 0x112);  // row_shr:2
+      VK_SCAN_ADD(d, 0x114);  // row_shr:4
+      VK_SCAN_ADD(d, 0x118);  // row_shr:8
+      l1[e] = __builtin_amdgcn_exp2f(d);   // Λ_t
+      rl[e] = __builtin_amdgcn_exp2f(-d);  // 1 / Λ_t
       l0[e] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, 1.0f),
-                                                                     __builtin_bit_cast(int, d), 0x111, 0xF, 0xF, false));
+                                                                     __builtin_bit_cast(int, l1[e]), 0x111, 0xF, 0xF, false));
     }
     float ah[4], rh[4], bh[4], kh[4], vv[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float rl = __builtin_amdgcn_rcpf(l1[e]);
       ah[e] = l0[e] * ((float)x.a[e] * in);
       rh[e] = l1[e] * ((float)x.r[e] * in);
-      bh[e] = ((float)x.b[e] * in) * rl;
-      kh[e] = ((float)x.k[e] * in) * rl;
+      bh[e] = ((float)x.b[e] * in) * rl[e];
+      kh[e] = ((float)x.k[e] * in) * rl[e];
       vv[e] = (float)x.v[e] * in;
     }
     *reinterpret_cast<fq4*>(&L.hat[b][0][ht][j0]) = fq4{ah[0], ah[1], ah[2], ah[3]};
@@ -1102,6 +1150,16 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra) {
           p1 = mfma4(a4[q][s2], st[q][s2], p1);
           y1 = mfma4(r4[q][s2], st[q][s2], y1);
         }
+      fq4 pm1 = {0.0f, 0.0f, 0.0f, 0.0f}, ym1 = pm1;
+      if constexpr (kSeg) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int s2 = 0; s2 < 4; ++s2) {
+            pm1 = mfma4(a4[q][s2], sm[q][s2], pm1);
+            ym1 = mfma4(r4[q][s2], sm[q][s2], ym1);
+          }
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -1114,39 +1172,71 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra) {
       fq4 z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int s2 = 0; s2 < 4; ++s2) z = mfma4(wt[s2], p1[s2], z);
+      fq4 zm = {0.0f, 0.0f, 0.0f, 0.0f};
+      if constexpr (kSeg) {
+#pragma unroll
+        for (int s2 = 0; s2 < 4; ++s2) zm = mfma4(wt[s2], pm1[s2], zm);
+      }
 #pragma unroll
       for (int s2 = 0; s2 < 4; ++s2) y1 = mfma4(trb[s2], z[s2], y1);
+      if constexpr (kSeg) {
+#pragma unroll
+        for (int s2 = 0; s2 < 4; ++s2) ym1 = mfma4(trb[s2], zm[s2], ym1);
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
 #pragma unroll
-        for (int s2 = 0; s2 < 4; ++s2) st[q] = mfma4(b4[q][s2], z[s2], st[q]);
+        for (int s2 = 0; s2 < 4; ++s2) {
+          st[q] = mfma4(b4[q][s2], z[s2], st[q]);
+          if constexpr (kSeg) sm[q] = mfma4(b4[q][s2], zm[s2], sm[q]);
+        }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) st[q][r] *= lamq[q][r];
+        for (int r = 0; r < 4; ++r) {
+          st[q][r] *= lamq[q][r];
+          if constexpr (kSeg) sm[q][r] *= lamq[q][r];
+        }
       }
-      // y rows t = 4 g + r of this wave's 16 value columns
-      _Float16 yh[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float yv = y1[r];
-        asm volatile("" : "+v"(yv));  // an fp32 value before the fp16 conversion
-        yh[r] = (_Float16)yv;
-      }
-      _Float16* yp = p.y + tok0 + (size_t)(c * kCL + 4 * g) * C + iw;
-      if (n == kCL) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) yp[(size_t)r * C] = yh[r];
-      } else {
+      if constexpr (kSeg) {
+        // outputs of N and M in fp32 (rows t = 4 g + r, this wave's 16 columns)
+        const size_t at = ((size_t)bi * sg.len + s0 + c * kCL + 4 * g) * C + (size_t)h * kHead + iw;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (4 * g + r < n) yp[(size_t)r * C] = yh[r];
+          if (4 * g + r < n) {
+            sg.y0[at + (size_t)r * C] = y1[r];
+            sg.q[at + (size_t)r * C] = ym1[r];
+          }
+      } else {
+        // y rows t = 4 g + r of this wave's 16 value columns
+        _Float16 yh[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float yv = y1[r];
+          asm volatile("" : "+v"(yv));  // an fp32 value before the fp16 conversion
+          yh[r] = (_Float16)yv;
+        }
+        _Float16* yp = p.y + tok0 + (size_t)(c * kCL + 4 * g) * C + iw;
+        if (n == kCL) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) yp[(size_t)r * C] = yh[r];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (4 * g + r < n) yp[(size_t)r * C] = yh[r];
+        }
       }
       // chunk c + 1's operands (past the last chunk: stale buffers, in bounds, never used)
       __builtin_amdgcn_sched_barrier(0);
       state_operands(c + 1);
       __syncthreads();
     }
+    float* const So = kSeg ? sg.n + (size_t)blockIdx.x * kHead * kHead : S;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) *reinterpret_cast<fq4*>(S + iw * kHead + 16 * q + 4 * g) = st[q];
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<fq4*>(So + iw * kHead + 16 * q + 4 * g) = st[q];
+    if constexpr (kSeg) {
+      float* const Mo = sg.m + (size_t)blockIdx.x * kHead * kHead;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) *reinterpret_cast<fq4*>(Mo + iw * kHead + 16 * q + 4 * g) = sm[q];
+    }
   } else {
     // The matrix waves' work is dependent chains (W^T's powers, LDS round trips, the Λ scans);
     // at a higher issue priority they go first whenever they can, and the state wave's
@@ -1168,6 +1258,147 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra) {
   }
 }
 
+// Step 2: one workgroup of 16 waves per chain, wave (ri, cj) the 16 x 16 tile of S = S M_p + N_p at
+// rows 16 ri, columns 16 cj.  S goes through LDS as the next product's A operand; the next
+// segment's M and N tiles are requested before the current products.
+template <bool kSlots>
+__global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(Fp32Args p, SegArgs sg) {
+  __shared__ __attribute__((aligned(16))) float s[kHead][kHP];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, g = lane >> 4, ri = w >> 2, cj = w & 3;
+  const int bh = blockIdx.x, bi = bh / p.H, h = bh - bi * p.H;
+  float* S = state_block<kSlots>(p, bi, h);
+  if (S == nullptr) return;
+  const size_t base = (size_t)bh * sg.P * kHead * kHead;
+  // B operand of k step (q, s2): M[16 q + 4 g + s2][16 cj + li]
+  float mb[2][16];
+  fq4 nt[2];
+  auto load = [&](int seg, int set) __attribute__((always_inline)) {
+    const float* M = sg.m + base + (size_t)seg * kHead * kHead + 16 * cj + li;
+    const float* N = sg.n + base + (size_t)seg * kHead * kHead + (16 * ri + 4 * g) * kHead + 16 * cj + li;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) mb[set][k] = M[(16 * (k >> 2) + 4 * g + (k & 3)) * kHead];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) nt[set][r] = N[r * kHead];
+  };
+  auto step = [&](int seg, int set) __attribute__((always_inline)) {
+    if (seg + 1 < sg.P) load(seg + 1, set ^ 1);
+    // S_start of this segment: thread -> 4 consecutive floats
+    *reinterpret_cast<fq4*>(sg.start + base + (size_t)seg * kHead * kHead + tid * 4) =
+        *reinterpret_cast<const fq4*>(&s[tid >> 4][4 * (tid & 15)]);
+    fq4 a[4], acc = nt[set];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const fq4*>(&s[16 * ri + li][16 * q + 4 * g]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int s2 = 0; s2 < 4; ++s2) acc = mfma4(a[q][s2], mb[set][4 * q + s2], acc);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s[16 * ri + 4 * g + r][16 * cj + li] = acc[r];
+    __syncthreads();
+  };
+  *reinterpret_cast<fq4*>(&s[tid >> 4][4 * (tid & 15)]) = *reinterpret_cast<const fq4*>(S + tid * 4);
+  load(0, 0);
+  __syncthreads();
+  for (int seg = 0; seg < sg.P; seg += 2) {
+    step(seg, 0);
+    if (seg + 1 < sg.P) step(seg + 1, 1);
+  }
+  *reinterpret_cast<fq4*>(S + tid * 4) = *reinterpret_cast<const fq4*>(&s[tid >> 4][4 * (tid & 15)]);
+}
+
+// Step 3: one workgroup per (chain, segment), wave w its chunks w, w + 4, ...: 16 tokens x 64
+// outputs each, S_start held in registers.
+template <bool kSlots>
+__global__ __launch_bounds__(256) void wkv_seg_out_kernel(Fp32Args p, SegArgs sg) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, g = lane >> 4;
+  const int bh = blockIdx.x / sg.P, seg = blockIdx.x - bh * sg.P, bi = bh / p.H, h = bh - bi * p.H;
+  const int C = p.C, s0 = seg * sg.cps * kCL, T = min(sg.len - s0, sg.cps * kCL);
+  _Float16* const y = p.y + ((size_t)bi * p.T + sg.t0 + s0) * C + (size_t)h * kHead;
+  if (state_block<kSlots>(p, bi, h) == nullptr) {
+    for (int idx = tid; idx < T * kHead; idx += 256) y[(size_t)(idx / kHead) * C + idx % kHead] = (_Float16)__builtin_nanf("");
+    return;
+  }
+  const float* S = sg.start + (size_t)blockIdx.x * kHead * kHead;
+  const size_t tok = ((size_t)bi * sg.len + s0) * C + (size_t)h * kHead;
+  fq4 sb[4][4];  // B operand of output tile c: S_start[16 c + li][16 q + 4 g ..]
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sb[c][q] = *reinterpret_cast<const fq4*>(S + (16 * c + li) * kHead + 16 * q + 4 * g);
+  for (int c0 = w * kCL; c0 < T; c0 += 4 * kCL) {
+    fq4 a[4], acc[4];
+    const float* qp = sg.q + tok + (size_t)min(c0 + li, T - 1) * C + 4 * g;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const fq4*>(qp + 16 * q);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* yp = sg.y0 + tok + (size_t)min(c0 + 4 * g + r, T - 1) * C + li;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c][r] = yp[16 * c];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int s2 = 0; s2 < 4; ++s2)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] = mfma4(a[q][s2], sb[c][q][s2], acc[c]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (c0 + 4 * g + r >= T) continue;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float v = acc[c][r];
+        asm volatile("" : "+v"(v));  // an fp32 value before the fp16 conversion
+        y[(size_t)(c0 + 4 * g + r) * C + 16 * c + li] = (_Float16)v;
+      }
+    }
+  }
+}
+
+// The segments of a prefill of T tokens of B sequences: P segments of cps chunks over blocks of
+// `len` tokens, or P = 1 (one chain per workgroup).
+struct SegPlan {
+  int P, cps, len;
+};
+
+constexpr int64_t kSegMaxBytes = (int64_t)96 << 20;  // of q and y0
+
+SegPlan seg_plan(int B, int T, int H) {
+  SegPlan one{1, 0, T};
+  const int64_t chains = (int64_t)B * H;
+  const int G = device_cus();
+  if (T < kChunkMinT || 2 * chains > G) return one;
+  const int64_t most = kSegMaxBytes / (chains * kHead * 8);  // tokens of a block
+  const int blocks = (int)((T + most - 1) / most);
+  const int len = ((T + blocks - 1) / blocks + kCL - 1) / kCL * kCL;
+  const int nchunk = (std::min(len, T) + kCL - 1) / kCL;
+  // Time model (us), both sides measured: one chain per workgroup 9.3 + 2.24 per chunk (T = 300: 52,
+  // T = 1500: 220); P segments 26 + 3.4 per chunk of a segment + 0.9 P (32 chains, T = 300, P = 6: 42;
+  // T = 1500, P = 8: 78; T = 4096: 587 -> 151; 128 chains, T = 1024, P = 2: 159 -> 145; below
+  // ~12 chunks the two extra launches cost more than they save: T = 128 27 against 32).
+  double best = 0.92 * (9.3 + 2.24 * nchunk);
+  SegPlan plan = one;
+  for (int P = 2; P <= G / chains && 2 * P <= nchunk; ++P) {
+    const int cps = (nchunk + P - 1) / P;
+    if ((nchunk + cps - 1) / cps != P) continue;
+    const double t = 26 + 3.4 * cps + 0.9 * P;
+    if (t < best) {
+      best = t;
+      plan = SegPlan{P, cps, std::min(len, T)};
+    }
+  }
+  return plan;
+}
+
+int64_t seg_bytes(const SegPlan& s, int B, int H) {
+  if (s.P == 1) return 0;
+  const int64_t chains = (int64_t)B * H;
+  return (chains * s.P * 3 * kHead * kHead + 2 * chains * s.len * kHead) * 4;
+}
+
 bool rows_vec_ok(const Fp32Args& p) {
   auto al = [](const void* x, uintptr_t m) { return ((uintptr_t)x & (m - 1)) == 0; };
   return al(p.r, 16) && al(p.w, 16) && al(p.k, 16) && al(p.v, 16) && al(p.a, 16) && al(p.b, 16) &&
@@ -1179,8 +1410,9 @@ bool rows_vec_ok(const Fp32Args& p) {
 // MI355X's memory-side cache (Infinity Cache).
 constexpr int64_t kMallBytes = (int64_t)256 << 20;
 
+// ws, ws_bytes: scratch for a segmented prefill (one chain per workgroup where it is too small).
 template <bool kSlots>
-void launch_fp32(const Fp32Args& p, int B, hipStream_t stream, bool rows) {
+void launch_fp32(const Fp32Args& p, int B, hipStream_t stream, bool rows, void* ws = nullptr, int64_t ws_bytes = 0) {
   if (p.T == 1) {
     const int64_t table = (int64_t)(kSlots ? p.n_slots : B) * p.H * kHead * kHead * 4;
     if (table > kMallBytes)
@@ -1189,9 +1421,24 @@ void launch_fp32(const Fp32Args& p, int B, hipStream_t stream, bool rows) {
       hipLaunchKernelGGL((wkv7_fp32_step_kernel<kSlots, false>), dim3(B * p.H), dim3(64), 0, stream, p);
   } else if (rows) {
     RowsArgs ra{p, rows_vec_ok(p) ? 1 : 0};
-    if (p.T >= kChunkMinT)
-      hipLaunchKernelGGL(wkv7_fp32_chunk_kernel<kSlots>, dim3(B * p.H), dim3(512), 0, stream, ra);
-    else if (ra.vec && B * p.H < 2 * device_cus())
+    if (p.T >= kChunkMinT) {
+      const SegPlan s = seg_plan(B, p.T, p.H);
+      if (s.P == 1 || ws == nullptr || ws_bytes < seg_bytes(s, B, p.H)) {
+        hipLaunchKernelGGL((wkv7_fp32_chunk_kernel<kSlots, false>), dim3(B * p.H), dim3(512), 0, stream, ra, SegArgs{});
+        return;
+      }
+      const int64_t mat = (int64_t)B * p.H * s.P * kHead * kHead;
+      float* f = reinterpret_cast<float*>(ws);
+      for (int t0 = 0; t0 < p.T; t0 += s.len) {
+        const int len = std::min(s.len, p.T - t0), nchunk = (len + kCL - 1) / kCL;
+        SegArgs sg{(nchunk + s.cps - 1) / s.cps, s.cps, t0, len, f, f + mat, f + 2 * mat, f + 3 * mat,
+                   f + 3 * mat + (int64_t)B * len * p.C};
+        const dim3 grid(B * p.H * sg.P);
+        hipLaunchKernelGGL((wkv7_fp32_chunk_kernel<kSlots, true>), grid, dim3(512), 0, stream, ra, sg);
+        hipLaunchKernelGGL(wkv_seg_chain_kernel<kSlots>, dim3(B * p.H), dim3(1024), 0, stream, p, sg);
+        hipLaunchKernelGGL(wkv_seg_out_kernel<kSlots>, grid, dim3(256), 0, stream, p, sg);
+      }
+    } else if (ra.vec && B * p.H < 2 * device_cus())
       hipLaunchKernelGGL((wkv7_fp32_rows_kernel<kSlots, 1>), dim3(2 * B * p.H), dim3(256), 0, stream, ra);
     else
       hipLaunchKernelGGL((wkv7_fp32_rows_kernel<kSlots, 2>), dim3(B * p.H), dim3(256), 0, stream, ra);
@@ -1718,6 +1965,39 @@ extern "C" int vkwr_wkv7_fp32_forward_slots(int B, int T, int C, int H, float* p
              reinterpret_cast<_Float16*>(y)};
   launch_fp32<true>(p, B, (hipStream_t)stream, true);
   return check_launch("vkwr_wkv7_fp32_forward_slots");
+}
+
+extern "C" int64_t vkwr_wkv7_fp32_prefill_workspace_bytes(int B, int T, int H) {
+  return B > 0 && T > 0 && H > 0 ? seg_bytes(seg_plan(B, T, H), B, H) : 0;
+}
+
+extern "C" int64_t vkwr_wkv7_fp32_prefill_workspace_max(int64_t rows, int H) {
+  if (rows <= 0 || H <= 0) return 0;
+  // the matrices of at most a segment per CU, and the rows of one block (a block's length is rounded
+  // up to whole chunks, of at most half a chain per CU)
+  const int64_t G = device_cus();
+  return (G * 3 * kHead * kHead) * 4 + std::min(rows * H * kHead * 8, kSegMaxBytes + G / 2 * kCL * kHead * 8);
+}
+
+extern "C" int vkwr_wkv7_fp32_prefill(int B, int T, int C, int H, float* state, int n_slots, const int32_t* slots,
+                                      const uint16_t* r, const uint16_t* w, const uint16_t* k, const uint16_t* v,
+                                      const uint16_t* a, const uint16_t* b, uint16_t* y, void* workspace,
+                                      int64_t workspace_bytes, void* stream) {
+  clear_error();
+  const char* fn = "vkwr_wkv7_fp32_prefill";
+  if (int e = check_wkv_dims(fn, B, T, C, H)) return e;
+  VK_REQUIRE(n_slots >= 0, "%s: negative pool size", fn);
+  if (B == 0 || H == 0 || T == 0) return VKWR_OK;
+  VK_REQUIRE(state && r && w && k && v && a && b && y, "%s: null pointer", fn);
+  if (((uintptr_t)workspace & 15) != 0) workspace = nullptr;  // 16-byte accesses: run without
+  Fp32Args p{T, C, H, slots ? n_slots : B, state, slots,
+             reinterpret_cast<const _Float16*>(r), reinterpret_cast<const _Float16*>(w),
+             reinterpret_cast<const _Float16*>(k), reinterpret_cast<const _Float16*>(v),
+             reinterpret_cast<const _Float16*>(a), reinterpret_cast<const _Float16*>(b),
+             reinterpret_cast<_Float16*>(y)};
+  if (slots) launch_fp32<true>(p, B, (hipStream_t)stream, true, workspace, workspace_bytes);
+  else launch_fp32<false>(p, B, (hipStream_t)stream, true, workspace, workspace_bytes);
+  return check_launch(fn);
 }
 
 extern "C" int vkwr_wkv7_fp32_step_rows_slots(int B, int C, int H, float* pool, int n_slots,
