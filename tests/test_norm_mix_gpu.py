@@ -231,6 +231,25 @@ def test_token_shift_prev_is_entry_value_for_long_prefill(gpu):
     assert np.array_equal(shift.cpu().numpy(), x[:, -1])
 
 
+@pytest.mark.parametrize("n_mix", [1, 6])
+@pytest.mark.parametrize("B,T,C", [(1, 2, 72), (2, 5, 64), (3, 4, 70), (40, 9, 2048), (130, 3, 2048), (9, 8, 24576)])
+def test_token_shift_runs(gpu, n_mix, B, T, C):
+    """Runs of 2 and of 4 tokens, whole and with a remainder, vector and scalar: mix = 1 gives the
+    previous token and mix = 0 the token itself, exactly (values whose difference is exact)."""
+    from vkwr._ops.v1 import v1_mix_ops as M
+    x, shift0 = ((np.round(h(*s) * 8) / 8).clip(-4, 4).astype(np.float16) for s in ((B, T, C), (B, C)))
+    shift, xd = dev(shift0, gpu), dev(x, gpu)
+    ones, zeros = dev(np.ones(C, np.float16), gpu), dev(np.zeros(C, np.float16), gpu)
+    if n_mix == 6:
+        outs = M.tmix_mix6(B, T, C, xd, shift, ones, zeros, ones, zeros, zeros, ones)
+    else:
+        outs = [M.cmix_mix(B, T, C, xd, shift, ones)]
+    prev = np.concatenate([shift0[:, None], x[:, :-1]], 1)
+    for o, want in zip(outs, (prev, x, prev, x, x, prev)):
+        assert np.array_equal(o.cpu().numpy(), want)
+    assert np.array_equal(shift.cpu().numpy(), x[:, -1])
+
+
 @pytest.mark.parametrize("half_math", [False, True])
 def test_tmix_mix6_t1_c4096(gpu, half_math):
     from vkwr._ops.v1 import v1_mix_ops as M

@@ -4,8 +4,7 @@
 // elementwise activations.  All HBM-bound.
 //
 // Token shift.  A lane owns 8 consecutive channels (one 16-byte access) of one
-// sequence for a run of up to kTokRun tokens, so x[t-1] is reused from
-// registers.  shift_state[b] is read (the previous token at t = 0) and then
+// sequence for a run of 2 or 4 tokens, so x[t-1] is reused from registers.  shift_state[b] is read (the previous token at t = 0) and then
 // overwritten with x[b,T-1] by the same lane -- the lane whose run starts at
 // t = 0 -- so prev at t = 0 is always the value at entry.  Algorithmic bytes
 // per token and channel: 2 (x) + 2n (outputs), plus 4 per sequence and
@@ -21,8 +20,6 @@
 namespace vk {
 namespace {
 
-constexpr int kTokRun = 16;
-
 struct ShiftArgs {
   int B, T, C;
   const _Float16* x;
@@ -33,11 +30,12 @@ struct ShiftArgs {
   _Float16* out[6];
 };
 
-// VW = 8 (16-byte accesses) or 1 (scalar); NMIX = 1 or 6.
-template <int VW, int NMIX, bool kHalfMath>
+// VW = 8 (16-byte accesses) or 1 (scalar); NMIX = 1 or 6; TR: tokens per run.  The rows of a run
+// are all requested before the first is used (rows past T are read clamped and dropped).
+template <int VW, int NMIX, bool kHalfMath, int TR>
 __global__ __launch_bounds__(256) void token_shift_kernel(ShiftArgs p) {
   const int nch = p.C / VW;
-  const int runs = (p.T + kTokRun - 1) / kTokRun;
+  const int runs = (p.T + TR - 1) / TR;
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= (int64_t)p.B * runs * nch) return;
   const int ch = (int)(gid % nch);
@@ -45,71 +43,64 @@ __global__ __launch_bounds__(256) void token_shift_kernel(ShiftArgs p) {
   const int run = (int)(rest % runs);
   const int b = (int)(rest / runs);
   const int c0 = ch * VW;
-  const int t0 = run * kTokRun;
-  const int t1 = min(p.T, t0 + kTokRun);
+  const int t0 = run * TR;
 
-  _Float16 mu[NMIX][VW];
-#pragma unroll
-  for (int i = 0; i < NMIX; ++i)
-#pragma unroll
-    for (int e = 0; e < VW; ++e) mu[i][e] = p.mix[i][c0 + e];
-
-  _Float16 prev[VW];
   const int64_t slot = p.shift_slots ? (int64_t)p.shift_slots[b] : b;
   const int64_t srow = slot * p.C + c0;
   const _Float16* xs = p.x + ((int64_t)b * p.T) * p.C + c0;
   if (p.shift_slots && (slot < 0 || slot >= p.n_slots)) {
     // A slot outside the pool: this sequence's outputs are NaN and no shift row is touched.
-    for (int t = t0; t < t1; ++t)
+    for (int t = t0; t < min(p.T, t0 + TR); ++t)
 #pragma unroll
       for (int i = 0; i < NMIX; ++i)
 #pragma unroll
         for (int e = 0; e < VW; ++e) p.out[i][((int64_t)b * p.T + t) * p.C + c0 + e] = (_Float16)__builtin_nanf("");
     return;
   }
-  if (t0 == 0) {
+  struct Row {
+    _Float16 v[VW];
+  };
+  auto ld = [](const _Float16* src) __attribute__((always_inline)) {
+    Row r;
+    if constexpr (VW == 8) *reinterpret_cast<h8*>(r.v) = ld8(src);
+    else r.v[0] = src[0];
+    return r;
+  };
+  Row row[TR + 1];  // row[u]: the token before t0 + u
+  row[0] = ld(t0 == 0 ? p.shift + srow : xs + (int64_t)(t0 - 1) * p.C);
 #pragma unroll
-    for (int e = 0; e < VW; ++e) prev[e] = p.shift[srow + e];
-  } else {
+  for (int u = 0; u < TR; ++u) row[u + 1] = ld(xs + (int64_t)min(t0 + u, p.T - 1) * p.C);
+  Row mu[NMIX];
 #pragma unroll
-    for (int e = 0; e < VW; ++e) prev[e] = xs[(int64_t)(t0 - 1) * p.C + e];
-  }
-  for (int t = t0; t < t1; ++t) {
-    _Float16 cur[VW];
-    const int64_t off = (int64_t)t * p.C;
-    if constexpr (VW == 8) {
-      *reinterpret_cast<h8*>(cur) = ld8(xs + off);
-    } else {
-      cur[0] = xs[off];
-    }
+  for (int i = 0; i < NMIX; ++i) mu[i] = ld(p.mix[i] + c0);
+  // This lane read the shift row above; it alone writes the new value.
+  Row last;
+  if (t0 == 0) last = ld(xs + (int64_t)(p.T - 1) * p.C);
+#pragma unroll
+  for (int u = 0; u < TR; ++u) {
+    if (t0 + u >= p.T) break;
 #pragma unroll
     for (int i = 0; i < NMIX; ++i) {
-      _Float16 o[VW];
+      Row o;
 #pragma unroll
       for (int e = 0; e < VW; ++e) {
+        const _Float16 prev = row[u].v[e], cur = row[u + 1].v[e];
         if constexpr (kHalfMath) {
-          const _Float16 dx = prev[e] - cur[e];
-          o[e] = (_Float16)__builtin_fmaf16(dx, mu[i][e], cur[e]);
+          const _Float16 dx = prev - cur;
+          o.v[e] = (_Float16)__builtin_fmaf16(dx, mu[i].v[e], cur);
         } else {
-          const float cf = (float)cur[e];
-          o[e] = f16_of(__builtin_fmaf((float)prev[e] - cf, (float)mu[i][e], cf));
+          const float cf = (float)cur;
+          o.v[e] = f16_of(__builtin_fmaf((float)prev - cf, (float)mu[i].v[e], cf));
         }
       }
-      _Float16* dst = p.out[i] + ((int64_t)b * p.T + t) * p.C + c0;
-      if constexpr (VW == 8) {
-        st8(dst, *reinterpret_cast<const h8*>(o));
-      } else {
-        dst[0] = o[0];
-      }
+      _Float16* dst = p.out[i] + ((int64_t)b * p.T + t0 + u) * p.C + c0;
+      if constexpr (VW == 8) st8(dst, *reinterpret_cast<const h8*>(o.v));
+      else dst[0] = o.v[0];
     }
-#pragma unroll
-    for (int e = 0; e < VW; ++e) prev[e] = cur[e];
   }
   if (t0 == 0) {
-    // This lane read shift_state above; it alone writes the new value.
-    const _Float16* last = xs + (int64_t)(p.T - 1) * p.C;
-#pragma unroll
-    for (int e = 0; e < VW; ++e) p.shift[srow + e] = last[e];
+    if constexpr (VW == 8) st8(p.shift + srow, *reinterpret_cast<const h8*>(last.v));
+    else p.shift[srow] = last.v[0];
   }
 }
 
@@ -323,10 +314,23 @@ int grid_for(int64_t items, const char* fn, unsigned* blocks) {
   return VKWR_OK;
 }
 
+template <int VW, int NMIX, int TR>
+int launch_shift_run(const ShiftArgs& p, bool half, const char* fn, hipStream_t s) {
+  unsigned blocks;
+  if (int e = grid_for((int64_t)p.B * ((p.T + TR - 1) / TR) * (p.C / VW), fn, &blocks)) return e;
+  if (half) hipLaunchKernelGGL((token_shift_kernel<VW, NMIX, true, TR>), dim3(blocks), dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((token_shift_kernel<VW, NMIX, false, TR>), dim3(blocks), dim3(256), 0, s, p);
+  return VKWR_OK;
+}
+
 template <int VW, int NMIX>
-void launch_shift(const ShiftArgs& p, bool half, unsigned blocks, hipStream_t s) {
-  if (half) hipLaunchKernelGGL((token_shift_kernel<VW, NMIX, true>), dim3(blocks), dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((token_shift_kernel<VW, NMIX, false>), dim3(blocks), dim3(256), 0, s, p);
+int launch_shift(const ShiftArgs& p, bool half, const char* fn, hipStream_t s) {
+  // Short runs fill the CUs and put all of a lane's rows in flight; long ones re-read less.  With
+  // runs of 16 walked row by row: T = 700, C = 2048, one mix 8.3 us (TR = 4 5-8, TR = 2 7.3); T = 50, six
+  // mixes 11.2 (TR = 2 4.5); 3 x 333, six mixes 13.5 (TR = 4 7.9); 8 x 1024, six mixes 38.7 (TR = 4 37.9).
+  const int64_t lanes4 = (int64_t)p.B * ((p.T + 3) / 4) * (p.C / VW);
+  if (lanes4 < 32768) return launch_shift_run<VW, NMIX, 2>(p, half, fn, s);
+  return launch_shift_run<VW, NMIX, 4>(p, half, fn, s);
 }
 
 }  // namespace
@@ -357,20 +361,11 @@ int token_shift_mix(const char* fn, int B, int T, int C, const uint16_t* x, uint
     p.out[i] = reinterpret_cast<_Float16*>(out[i]);
     vec = vec && aligned16(mix[i]) && aligned16(out[i]);
   }
-  const int VW = vec ? 8 : 1;
-  const int64_t items = (int64_t)B * ((T + kTokRun - 1) / kTokRun) * (C / VW);
-  unsigned blocks;
-  if (int e = grid_for(items, fn, &blocks)) return e;
   hipStream_t s = (hipStream_t)stream;
   const bool half = half_math != 0;
-  if (vec) {
-    if (n_mix == 1) launch_shift<8, 1>(p, half, blocks, s);
-    else launch_shift<8, 6>(p, half, blocks, s);
-  } else {
-    if (n_mix == 1) launch_shift<1, 1>(p, half, blocks, s);
-    else launch_shift<1, 6>(p, half, blocks, s);
-  }
-  return check_launch(fn);
+  const int e = vec ? (n_mix == 1 ? launch_shift<8, 1>(p, half, fn, s) : launch_shift<8, 6>(p, half, fn, s))
+                    : (n_mix == 1 ? launch_shift<1, 1>(p, half, fn, s) : launch_shift<1, 6>(p, half, fn, s));
+  return e ? e : check_launch(fn);
 }
 }  // namespace
 
