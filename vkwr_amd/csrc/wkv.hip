@@ -27,6 +27,7 @@
 // chunks per row, slot i*8 + (q ^ ((i >> 1) & 7))).
 
 #include <algorithm>
+#include <type_traits>
 
 #include "vk_capi.h"
 #include "vk_common.cuh"
@@ -1895,6 +1896,236 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   }
 }
 
+// The same recurrence for T > 1 with one workgroup per CU or fewer: four waves per (sequence,
+// head), so that a lone wave's 160 FMAs per token become ~90 on each of the four SIMDs.
+//
+// Wave w owns rows 16 w .. 16 w + 15; the four lanes of a quad hold one row, lane cg of it columns 16
+// cg .. 16 cg + 15.  The updates are local.  Each dot product keeps the reference's order (two
+// interleaved chains over the 64 columns): it passes through the column groups in turn, 8 FMAs
+// in each, all lanes executing every stage and only the lane whose turn it is holding the true
+// sum, which a quad broadcast hands on.  The y and the next token's sa chains run side by
+// side (a dependent packed FMA may issue every other slot).  Bit-exact against wkv7_fp16_kernel.
+//
+// The token vectors are staged 16 tokens at a time by all 256 threads (the decay once per token
+// and channel: 4 of its ~60 instructions per token and lane instead of 60), two buffers, two
+// barriers per 16 tokens; a token's vectors are read from LDS while the previous one computes.
+// What bounds it: one wave per SIMD and the chains' 64 dependent FMAs and hand-overs per
+// token.  B H = 64, T = 300: 200 -> 110 us (0.66 -> 0.36 us a token).
+constexpr int kF16TC = 16;  // tokens per staged chunk
+template <bool kLegacy>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void wkv7_fp16_quad_kernel(Fp16Args p) {
+  // [buffer][token][r, decay, k, a, b, v][channel]
+  __shared__ __attribute__((aligned(16))) _Float16 vec[2][kF16TC][6][kHead];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int cg = lane & 3;
+  const int bh = blockIdx.x, bi = bh / p.H, h = bh - bi * p.H;
+  const int T = p.T, row = 16 * w + (lane >> 2);
+  const size_t tok0 = (size_t)bi * T * p.C + (size_t)h * kHead;
+  _Float16* const Sp = p.state + (size_t)bh * (kHead * kHead) + row * kHead + 16 * cg;
+
+  h2 s[8];
+  *reinterpret_cast<hv8*>(&s[0]) = *reinterpret_cast<const hv8*>(Sp);
+  *reinterpret_cast<hv8*>(&s[4]) = *reinterpret_cast<const hv8*>(Sp + 8);
+
+  // staging: thread -> the decay of 4 channels of one token, and pieces tid, tid + 256, tid + 512
+  // (of 640) of the other five vectors
+  const uint32_t el = (uint32_t)p.elapsed[bi];
+  const int wt = tid >> 4, wc = 4 * (tid & 15);
+  typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
+  const bool has_w0 = !kLegacy && p.w0 != nullptr;
+  hv4 w0 = {};
+  if (has_w0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w0[e] = p.w0[h * kHead + wc + e];
+  }
+  const _Float16* const src[5] = {p.r, p.k, p.a, p.b, p.v};
+  constexpr int kSlot[5] = {0, 2, 3, 4, 5};
+  hv4 gw;
+  hv8 gp[3];
+  auto fetch = [&](int c) __attribute__((always_inline)) {
+    const int t0 = c * kF16TC;
+    gw = *reinterpret_cast<const hv4*>(p.w + tok0 + (size_t)min(t0 + wt, T - 1) * p.C + wc);
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const int i = min(tid + 256 * u, 639), v = i >> 7, t = (i >> 3) & 15;
+      gp[u] = *reinterpret_cast<const hv8*>(src[v] + tok0 + (size_t)min(t0 + t, T - 1) * p.C + (i & 7) * 8);
+    }
+  };
+  auto stage = [&](int c) __attribute__((always_inline)) {
+    auto& vb = vec[c & 1];
+    hv4 d;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float wf = (float)gw[e];
+      uint32_t phase = el + (uint32_t)(c * kF16TC + wt);
+      if constexpr (!kLegacy) {
+        if (has_w0) wf = wf + (float)w0[e];
+        phase += (uint32_t)(h * kHead + wc + e);
+      }
+      d[e] = w_delta(wf, phase);
+    }
+    *reinterpret_cast<hv4*>(&vb[wt][1][wc]) = d;
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const int i = tid + 256 * u;
+      if (i < 640) *reinterpret_cast<hv8*>(&vb[(i >> 3) & 15][kSlot[i >> 7]][(i & 7) * 8]) = gp[u];
+    }
+  };
+
+  struct Tok {
+    h2 r[8], w[8], k[8], b[8];
+    _Float16 v;
+  };
+  auto rd = [&](int t, int slot, h2 (&x)[8]) __attribute__((always_inline)) {
+    const _Float16* at = &vec[(t >> 4) & 1][t & 15][slot][16 * cg];
+    *reinterpret_cast<hv8*>(&x[0]) = *reinterpret_cast<const hv8*>(at);
+    *reinterpret_cast<hv8*>(&x[4]) = *reinterpret_cast<const hv8*>(at + 8);
+  };
+  auto read_tok = [&](int t, Tok& x) __attribute__((always_inline)) {
+    rd(t, 0, x.r);
+    rd(t, 1, x.w);
+    rd(t, 2, x.k);
+    rd(t, 4, x.b);
+    x.v = vec[(t >> 4) & 1][t & 15][5][row];
+  };
+  // lane k of every quad to the whole quad
+  auto from = [](h2 x, auto k) __attribute__((always_inline)) {
+    constexpr int kCtrl = decltype(k)::value * 0x55;
+    return __builtin_bit_cast(h2, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), kCtrl, 0xF, 0xF, true));
+  };
+  using K0 = std::integral_constant<int, 0>;
+  using K1 = std::integral_constant<int, 1>;
+  using K2 = std::integral_constant<int, 2>;
+  using K3 = std::integral_constant<int, 3>;
+  const h2 zero = {(_Float16)0.0f, (_Float16)0.0f};
+  auto chain = [](const h2 (&x)[8], const h2 (&c)[8], h2 acc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      if constexpr (kLegacy) acc = acc + x[m] * c[m];
+      else acc = __builtin_elementwise_fma(x[m], c[m], acc);
+    }
+    return acc;
+  };
+  // both chains one stage at a time, interleaved FMA by FMA
+  auto chain2 = [](const h2 (&x)[8], const h2 (&r)[8], const h2 (&a)[8], h2& y, h2& n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      if constexpr (kLegacy) {
+        y = y + x[m] * r[m];
+        n = n + a[m] * x[m];
+      } else {
+        y = __builtin_elementwise_fma(x[m], r[m], y);
+        n = __builtin_elementwise_fma(a[m], x[m], n);
+      }
+    }
+  };
+  auto sum = [](h2 x) __attribute__((always_inline)) {
+    const _Float16 v = x.x + x.y;
+    return h2{v, v};
+  };
+
+  fetch(0);
+  stage(0);
+  fetch(1);
+  __syncthreads();
+  Tok x0, x1;
+  h2 a0[8], a1[8];
+  read_tok(0, x0);
+  rd(0, 3, a0);
+  h2 sav;
+  {
+    h2 n = chain(s, a0, zero);
+    n = chain(s, a0, from(n, K0{}));
+    n = chain(s, a0, from(n, K1{}));
+    n = chain(s, a0, from(n, K2{}));
+    sav = from(sum(n), K3{});
+  }
+  rd(1, 3, a0);
+
+  // token t (vectors in x; a: the next token's a); reads token t + 1's vectors into nx and token
+  // t + 2's a into na
+  auto token = [&](int t, const Tok& x, const h2 (&a)[8], Tok& nx, h2 (&na)[8]) __attribute__((always_inline)) {
+    // The LDS reads go out two at a time between the FMAs: the four waves run in step, and their 40
+    // reads of 1 KiB at once held each wave up for as long as the LDS took (380 -> 366 ns a token).
+    const auto reads = [&](auto step) __attribute__((always_inline)) {
+      constexpr int kStep = decltype(step)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kStep == 0) rd(t + 1, 4, nx.b);
+      if constexpr (kStep == 1) rd(t + 1, 2, nx.k);
+      if constexpr (kStep == 2) rd(t + 1, 1, nx.w);
+      if constexpr (kStep == 3) rd(t + 1, 0, nx.r);
+      if constexpr (kStep == 4) rd(t + 2, 3, na);
+      if constexpr (kStep == 5) nx.v = vec[((t + 1) >> 4) & 1][(t + 1) & 15][5][row];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    const h2 vv = {x.v, x.v};
+    // (the updates in three sweeps, so that no FMA waits for the one before it)
+    h2 in[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      if constexpr (kLegacy) in[m] = s[m] * x.w[m];
+      else in[m] = __builtin_elementwise_fma(sav, x.b[m], s[m]);
+    }
+    reads(K0{});
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      if constexpr (kLegacy) {
+        const h2 t2 = x.k[m] * vv;
+        const h2 t3 = in[m] + t2;
+        const h2 t4 = sav * x.b[m];
+        in[m] = t3 + t4;
+      } else {
+        in[m] = __builtin_elementwise_fma(x.k[m], vv, in[m]);
+      }
+    }
+    reads(K1{});
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      if constexpr (kLegacy) s[m] = s[m] + in[m];
+      else s[m] = __builtin_elementwise_fma(s[m], x.w[m], in[m]);
+    }
+    reads(K2{});
+    h2 y = zero, n = zero;
+    chain2(s, x.r, a, y, n);
+    y = from(y, K0{});
+    n = from(n, K0{});
+    reads(K3{});
+    chain2(s, x.r, a, y, n);
+    y = from(y, K1{});
+    n = from(n, K1{});
+    reads(std::integral_constant<int, 4>{});
+    reads(std::integral_constant<int, 5>{});
+    chain2(s, x.r, a, y, n);
+    y = from(y, K2{});
+    n = from(n, K2{});
+    chain2(s, x.r, a, y, n);
+    sav = from(sum(n), K3{});
+    _Float16 yv = y.x + y.y;
+    asm volatile("" : "+v"(yv));  // all of the chain stays outside the branch
+    if (cg == 3) p.y[tok0 + (size_t)t * p.C + row] = yv;
+  };
+
+  // (the vectors read past token T - 1 are stale or clamped copies, in bounds and never used)
+  const int nchunk = (T + kF16TC - 1) / kF16TC;
+  for (int c = 0; c < nchunk; ++c) {
+    const int t0 = c * kF16TC, n = min(kF16TC, T - t0);
+    stage(c + 1);  // its buffer was last read before the barrier that ended chunk c - 1
+    fetch(c + 2);
+    for (int u = 0; u < 8; u += 2) {
+      if (u < n) token(t0 + u, x0, a0, x1, a1);
+      if (u + 1 < n) token(t0 + u + 1, x1, a1, x0, a0);
+    }
+    __syncthreads();  // chunk c + 1 is staged
+    for (int u = 8; u < kF16TC; u += 2) {
+      if (u < n) token(t0 + u, x0, a0, x1, a1);
+      if (u + 1 < n) token(t0 + u + 1, x1, a1, x0, a0);
+    }
+    __syncthreads();  // chunk c's buffer is free
+  }
+  *reinterpret_cast<hv8*>(Sp) = *reinterpret_cast<const hv8*>(&s[0]);
+  *reinterpret_cast<hv8*>(Sp + 8) = *reinterpret_cast<const hv8*>(&s[4]);
+}
+
 __global__ __launch_bounds__(256) void advance_i32_kernel(int32_t* x, int64_t n, int32_t amount) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] = (int32_t)((uint32_t)x[i] + (uint32_t)amount);
@@ -2083,7 +2314,15 @@ static int launch_fp16(const char* fn, bool legacy, int B, int T, int C, int H, 
              reinterpret_cast<const _Float16*>(b), reinterpret_cast<_Float16*>(y), elapsed_t};
   // T > 1 with at most one wave per SIMD: the latency-scheduled form (same arithmetic)
   const bool seq = T > 1 && (int64_t)B * H <= 4 * (int64_t)device_cus();
-  if (legacy) {
+  // ... and four waves per chain where each has a CU to itself and the rows are 16-byte aligned: T = 300,
+  // 256 chains 201 -> 117 us; two to a CU lose (288 chains 198 us with one wave, 218 with four; 512: 201, 226)
+  auto al = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
+  const bool quad = T > 1 && (int64_t)B * H <= (int64_t)device_cus() && al(state) && al(r) && al(w) && al(k) &&
+                    al(v) && al(a) && al(b);
+  if (quad) {
+    if (legacy) hipLaunchKernelGGL(wkv7_fp16_quad_kernel<true>, dim3(B * H), dim3(256), 0, (hipStream_t)stream, p);
+    else hipLaunchKernelGGL(wkv7_fp16_quad_kernel<false>, dim3(B * H), dim3(256), 0, (hipStream_t)stream, p);
+  } else if (legacy) {
     if (seq) hipLaunchKernelGGL(wkv7_fp16_seq_kernel<true>, dim3(B * H), dim3(64), 0, (hipStream_t)stream, p);
     else hipLaunchKernelGGL(wkv7_fp16_kernel<true>, dim3(B * H), dim3(64), 0, (hipStream_t)stream, p);
   } else {
