@@ -20,7 +20,7 @@ def _at_offset(x, off):
 
 
 @pytest.mark.parametrize("variant", ["seq", "w0", "legacy"])
-@pytest.mark.parametrize("B,T,H,odd", [(1, 2, 1, None), (2, 15, 3, None), (1, 16, 2, None), (3, 17, 2, None),
+@pytest.mark.parametrize("B,T,H,odd", [(1, 4, 1, None), (1, 3, 1, None), (2, 15, 3, None), (1, 16, 2, None), (3, 17, 2, None),
                                        (1, 33, 5, None), (2, 19, 2, "y"), (2, 19, 2, "v"), (2, 19, 2, "w"),
                                        (17, 18, 32, None)])
 def test_bits(gpu, variant, B, T, H, odd):

@@ -2315,9 +2315,10 @@ static int launch_fp16(const char* fn, bool legacy, int B, int T, int C, int H, 
   // T > 1 with at most one wave per SIMD: the latency-scheduled form (same arithmetic)
   const bool seq = T > 1 && (int64_t)B * H <= 4 * (int64_t)device_cus();
   // ... and four waves per chain where each has a CU to itself and the rows are 16-byte aligned: T = 300,
-  // 256 chains 201 -> 117 us; two to a CU lose (288 chains 198 us with one wave, 218 with four; 512: 201, 226)
+  // 256 chains 201 -> 117 us; two to a CU lose (288 chains 198 us with one wave, 218 with four; 512: 201, 226),
+  // and from T = 4 (8 sequences of 2 tokens 7.7 us with one wave, 8.7 with four; 2 of 4: 8.8, 8.7)
   auto al = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-  const bool quad = T > 1 && (int64_t)B * H <= (int64_t)device_cus() && al(state) && al(r) && al(w) && al(k) &&
+  const bool quad = T >= 4 && (int64_t)B * H <= (int64_t)device_cus() && al(state) && al(r) && al(w) && al(k) &&
                     al(v) && al(a) && al(b);
   if (quad) {
     if (legacy) hipLaunchKernelGGL(wkv7_fp16_quad_kernel<true>, dim3(B * H), dim3(256), 0, (hipStream_t)stream, p);
