@@ -39,6 +39,9 @@ def run(a, w, layout, gpu, act=None, epi=capi.EPI_NONE, v=None, vf=None, v0=None
     (333, 480, 1000),      # a ragged last stage after whole ones
     (200, 2048, 2048),     # a whole K, ring wrapped several times
     (700, 8192, 264),      # K in 4 parts, partial planes and the reduce
+    (1000, 2048, 2048),    # 128 x 64 tiles, a ragged last row of tiles
+    (520, 2056, 2056),     # 128 x 64, ragged everywhere
+    (200, 8192, 2048),     # 128 x 64, K in 4 parts
     (2304, 4096, 512),     # 128 x 128 tiles, K in 3 parts
     (300, 2056, 8200),     # 128 x 128, ragged everywhere
     (1024, 256, 8192),     # 256 x 128, whole

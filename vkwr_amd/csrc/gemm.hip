@@ -2278,7 +2278,11 @@ double gemm_stream_us(const Batch& bt) {
 // workspace that takes.  Fitted to sweeps over M = 64..3000 and (K, N) from (96, 2048) to
 // (16384, 4096): a workgroup costs `over` (first loads, output) plus its stages; a stage takes
 // longer the more CUs are busy (L2 and fabric).  64 x 64 tiles sit two to a CU, the others one.
-//   64 x 64    M = 512, K = N = 2048 (256 tiles)          13.9 modelled, 10.4 measured
+//   64 x 64    M = 512, K = N = 2048 (256 tiles)          10.2 modelled, 10.4 measured
+//   128 x 64   M = 1000, K = N = 2048 (256 tiles)         15.0, 14.2 (64 x 64 there 16.9, 128 x 128 17.5)
+//              M = 200, K = 8192, N = 2048 (4 parts)      22 measured (28.5 with the other tiles)
+//              M = 160, K = 2048, N = 8192 (256 tiles)    15.0, 17.1 (128 x 128 there 20.2)
+//              M = 300, K = N = 4096 (192 tiles)          24.2, 27.9 (128 x 128 there 26.6: within the model's error)
 //   128 x 128  M = 2048, K = N = 2048 (256 tiles)         20.2, 19.6
 //   256 x 128  M = 512, K = 4096, N = 16384 (256 tiles)   66.2, 66.6
 double mid_estimate(const Batch& bt, int G, int bm, int bn, int parts, bool unequal, double floor_us, int64_t* ws,
@@ -2304,11 +2308,21 @@ double mid_estimate(const Batch& bt, int G, int bm, int bn, int parts, bool uneq
   *tiles = W;
   const int slots = two ? 2 * G : G;
   const double fill = std::min(1.0, (double)W / G);
-  const bool sq = bm == 128 && bn == 128;
-  const double t0 = two ? 3.2 : 1.8, over = two ? (W <= slots ? 0.6 : 2.1) : (sq ? 3.0 : 4.2);
-  double stage = two ? (W <= G ? 0.20 : 0.27 + 0.14 * std::min(1.0, (double)W / slots))
-                     : (sq ? (W <= G ? 0.36 + 0.16 * fill : 0.56) : 0.60 + 0.34 * fill);
-  if (bn == 256) stage *= 1.02;
+  double t0 = 1.8, over, stage;
+  if (two) {
+    t0 = 3.2;
+    over = W <= slots ? 0.6 : 2.1;
+    stage = W <= G ? 0.20 : 0.27 + 0.14 * std::min(1.0, (double)W / slots);
+  } else if (bn == 64) {
+    over = 2.6;
+    stage = 0.25 + 0.08 * fill;
+  } else if (bm == 128 && bn == 128) {
+    over = 3.0;
+    stage = W <= G ? 0.36 + 0.16 * fill : 0.56;
+  } else {
+    over = 4.2;
+    stage = (0.60 + 0.34 * fill) * (bn == 256 ? 1.02 : 1.0);
+  }
   const double act = 0.0066 * bm;  // a stage's activations: ~64 clocks per wave and value
   const double mean = over + (work * stage + acts * act) / W;
   double t = over + longest * (stage + (acts > 0 ? act : 0.0));
@@ -2370,7 +2384,7 @@ void mid_choose(Batch& bt, int max_m, int64_t limit, const BigPlan& pl, double p
   } else if (cfg.big) {
     base = big_estimate(bt, pl, planned);
   }
-  static const int shapes[4][2] = {{64, 64}, {128, 128}, {256, 128}, {128, 256}};
+  static const int shapes[5][2] = {{64, 64}, {128, 64}, {128, 128}, {256, 128}, {128, 256}};
   Config best = cfg;
   const double floor_us = gemm_stream_us(bt);
   const int G = device_cus();
@@ -2530,6 +2544,7 @@ void mid_launch_tile(bool kn, bool act, const Batch& bt, int wgs, hipStream_t s)
 
 void mid_launch(const Config& cfg, bool act, const Batch& bt, int wgs, hipStream_t s) {
   if (cfg.bm == 64) mid_launch_tile<64, 64, 4>(cfg.kn, act, bt, wgs, s);
+  else if (cfg.bn == 64) mid_launch_tile<128, 64, 4>(cfg.kn, act, bt, wgs, s);
   else if (cfg.bn == 256) mid_launch_tile<128, 256, 3>(cfg.kn, act, bt, wgs, s);
   else if (cfg.bm == 256) mid_launch_tile<256, 128, 3>(cfg.kn, act, bt, wgs, s);
   else mid_launch_tile<128, 128, 4>(cfg.kn, act, bt, wgs, s);
