@@ -523,7 +523,7 @@ typedef struct vkwr_frag_gemm_problem {
 VKWR_EXPORT int vkwr_frag_gemm_f16(int n_problems, const vkwr_frag_gemm_problem* problems,
                                    void* stream);
 
-/* One frag GEMM with K split over `splits` workgroups per 64 x 64 output
+/* One frag GEMM with K split over `splits` workgroups per output
  * tile: the parts write fp32 partial tiles to `workspace`, and a second
  * kernel adds them in increasing K order and applies the epilogue (same
  * epilogues and layouts as vkwr_frag_gemm_f16).  For long-K decode GEMMs

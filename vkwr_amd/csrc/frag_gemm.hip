@@ -22,7 +22,7 @@
 //    Deterministic, no second kernel, no fp32 partials in HBM.
 //
 //  * For long K (the FFN value, K = 4 C) the same kernel can instead give
-//    each workgroup one K part of a 64 x 64 tile and write its fp32 partial
+//    each workgroup one K part of a tile (64 x 64 at 33 - 128 rows) and write its fp32 partial
 //    tile to a caller workspace (vkwr_frag_gemm_splitk_f16): each workgroup
 //    then reads half the activation bytes of the unsplit 32 x 32 form, and
 //    frag_splitk_reduce_kernel (or the consumer) adds the parts in K order.
@@ -57,8 +57,9 @@ struct FProb {
   int epi, c_frag;
   int ncol, nmb;            // column tiles, row tiles
   int wg_begin;             // first workgroup id (multiple of 8)
-  float* ws;                // K split: fp32 partial tiles [ksplit][nmb * 32 * TM][npad]
+  float* ws;                // K split: fp32 partial planes [ksplit][ws_rows][npad]
   int ksplit;               // K parts (1: no split)
+  int ws_rows;              // rows of a part's plane
   int xcd_map;              // row tiles of a column tile share an XCD
 };
 
@@ -187,9 +188,9 @@ __global__ __launch_bounds__(NW * 64) void frag_gemm_kernel(FBatch bt) {
   const int m = Pr.m, n = Pr.n, npad = Pr.npad, kpad = Pr.kpad, epi = Pr.epi, c_frag = Pr.c_frag;
   const int ncol = Pr.ncol, nmb = Pr.nmb, xcd_map = Pr.xcd_map, wg_begin = Pr.wg_begin;
   float* const ws = Pr.ws;
-  const int ksplit = kStore == kStorePartial ? Pr.ksplit : 1;
+  const int ksplit = kStore == kStorePartial ? Pr.ksplit : 1, ws_rows = Pr.ws_rows;
   asm volatile("" ::"s"(pa), "s"(pb), "s"(pc), "s"(pv), "s"(pvf), "s"(pv0), "s"(m), "s"(n), "s"(npad), "s"(kpad),
-               "s"(epi), "s"(c_frag), "s"(ncol), "s"(nmb), "s"(xcd_map), "s"(wg_begin), "s"(ws), "s"(ksplit));
+               "s"(epi), "s"(c_frag), "s"(ncol), "s"(nmb), "s"(xcd_map), "s"(wg_begin), "s"(ws), "s"(ksplit), "s"(ws_rows));
   const int lt = (int)blockIdx.x - wg_begin;
   if (lt >= ncol * nmb * ksplit) return;  // round-up workgroup
   // Tile and K part.  With the XCD map, the K parts and row tiles of a column
@@ -297,7 +298,8 @@ __global__ __launch_bounds__(NW * 64) void frag_gemm_kernel(FBatch bt) {
     const int row = (mb * TM + i) * 32 + 8 * (r >> 2) + 4 * (l0 >> 5) + (r & 3);
     const int col = (cb * TN + j) * 32 + (l0 & 31);
     if constexpr (kStore == kStorePartial) {
-      float* const o = ws + ((int64_t)part * nmb * (32 * TM) + row) * npad + col;
+      if (row >= ws_rows) continue;  // (a 128-row tile's lower half)
+      float* const o = ws + ((int64_t)part * ws_rows + row) * npad + col;
       *reinterpret_cast<f4*>(o) = s0;
       *reinterpret_cast<f4*>(o + 4) = s1;
       continue;
@@ -378,31 +380,54 @@ int tiles_for(const FBatch& bt, int bm, int bn) {
   return t;
 }
 
-// One configuration per launch.  Large batches of tiles take 128 x 64 tiles;
-// medium ones 64 x 64; small ones (fewer than 128 such tiles: too few
-// workgroups for 256 CUs) 32 x 32 with more K per block.
-FragConfig pick_frag_config(const FBatch& bt) {
-  int max_m = 0;
+// One configuration per launch; `splits` K parts per tile.
+//
+// The smallest tile whose workgroups fit the 256 CUs at once: a second round of workgroups costs more
+// than larger tiles that leave some CUs idle, and half as many workgroups as CUs leave bandwidth.
+// us, this tile against the others (proj: three [C, C] and four low-rank problems in a launch):
+//   32 x 32    K 2048, N 8192, m <= 32    8.9; 32 x 64 11.0, 64 x 64 12.8
+//   32 x 64    the same, m = 64          11.2; 64 x 64 13.4, 32 x 32 12.8
+//              K = N = 2048, m = 160      6.6; 32 x 32 7.6
+//   64 x 64    K 2048, N 8192, m = 128   13.1; 32 x 64 15.0
+//   128 x 64   the same, m = 160 - 256   17.0; 64 x 64 20.9
+//              K 4096, N 16384, m = 80   36.7; 64 x 64 43.8
+//              proj, C 4096, m = 128     38.7; 64 x 64 44.4
+// K up to 1024: up to three rounds of 32 x 32, several to a CU, cost less than one of larger tiles (proj,
+// C 768, m = 160: 6.3, 64 x 64 7.8, 32 x 64 9.3; m = 256: 7.4, 64 x 64 7.8; K 768, N 3072, m = 256: 5.7, 5.5).
+//
+// Beyond one round of 128 x 64: 64 x 64 with four waves, two to a CU, where 128-row tiles would pad more
+// rows (K 2048, N 65536, m = 129: 101, 128 x 64 121; K 4096, N 16384, m = 160: 53, 57.5) or K is short (K 768,
+// N 65536, m = 128: 34, 38); 128 x 64 otherwise (K 4096, N 16384, m = 256: 58, 66).
+//
+// K up to 512 (the low-rank outputs): a workgroup lives for one to four loads, so many small
+// ones side by side hide each other's start (four of N 2048, m = 128: 32 x 64 with four waves 4.5, 64 x 64
+// with eight 4.9; m = 256: 5.4, 9.1 with 128 x 64; N 4096, m = 128: 5.4, 9.1).
+FragConfig pick_frag_config(const FBatch& bt, int splits) {
+  int max_m = 0, max_k = 0;
   int64_t kdiv = 0;  // gcd of the padded K
   for (int i = 0; i < bt.n; ++i) {
     max_m = std::max(max_m, bt.p[i].m);
+    max_k = std::max(max_k, bt.p[i].kpad);
     int64_t a = kdiv, b = bt.p[i].kpad;
     while (b) { const int64_t t = a % b; a = b; b = t; }
     kdiv = a;
   }
+  kdiv /= splits;
   auto ks_for = [&](int nw, int ks_max) {
     int ks = ks_max;
     while (ks > 1 && kdiv % (16 * ks * nw) != 0) ks /= 2;
     return ks;
   };
-  if (max_m <= 32) {
-    if (tiles_for(bt, 32, 64) >= 128) return {1, 2, 8, ks_for(8, 2)};
-    return {1, 1, 8, ks_for(8, 4)};
-  }
-  const int t64 = tiles_for(bt, 64, 64);
-  if (t64 >= 1024) return {4, 2, 4, 2};
-  if (t64 >= 128) return {2, 2, 8, ks_for(8, 2)};
-  return {1, 1, 8, ks_for(8, 4)};
+  auto fits = [&](int bm, int bn) { return (int64_t)tiles_for(bt, bm, bn) * splits <= 256; };
+  if (fits(32, 32)) return {1, 1, 8, ks_for(8, 4)};
+  if (splits == 1 && max_k <= 512) return {1, 2, 4, 1};
+  if (splits == 1 && max_k <= 1024 && tiles_for(bt, 32, 32) <= 768) return {1, 1, 8, ks_for(8, 4)};
+  if (fits(32, 64)) return {1, 2, 8, ks_for(8, 2)};
+  if (fits(64, 64)) return {2, 2, 8, ks_for(8, 2)};
+  if (fits(128, 64)) return {4, 2, 4, ks_for(4, 2)};
+  if (max_m <= 32) return {1, 2, 8, ks_for(8, 2)};
+  if (splits == 1 && (max_k <= 1024 || tiles_for(bt, 64, 64) < 2 * tiles_for(bt, 128, 64))) return {2, 2, 4, 2};
+  return {4, 2, 4, ks_for(4, 2)};
 }
 
 // One workgroup range per problem, each a multiple of 8 long (so a tile's id
@@ -442,6 +467,8 @@ int launch_frag(const FBatch& bt, FragConfig c, int wgs, hipStream_t s) {
     return VKWR_OK;                                                       \
   }
   VK_FRAG_CASE(4, 2, 4, 2)
+  VK_FRAG_CASE(2, 2, 4, 2)
+  VK_FRAG_CASE(1, 2, 4, 1)
   VK_FRAG_CASE(2, 2, 8, 2)
   VK_FRAG_CASE(2, 2, 8, 1)
   VK_FRAG_CASE(1, 1, 8, 4)
@@ -534,8 +561,13 @@ int fill_problem(const char* fn, int i, const vkwr_frag_gemm_problem& q, FProb& 
   return VKWR_OK;
 }
 
-// The K-split GEMM runs on 64 x 64 tiles, 8 waves, two 16-k steps per load.
+// A K-split GEMM's planes hold rows in multiples of 64, and a part two 16-k steps of eight waves.
 constexpr int kSplitTile = 64, kSplitKRound = 16 * 2 * 8;
+
+template <int TM, int TN, int NW, int KS>
+void launch_partial(const FBatch& bt, int wgs, hipStream_t s) {
+  hipLaunchKernelGGL((frag_gemm_kernel<TM, TN, NW, KS, kStorePartial, false>), dim3(wgs), dim3(NW * 64), 0, s, bt);
+}
 
 }  // namespace
 
@@ -553,7 +585,7 @@ extern "C" int vkwr_frag_gemm_f16(int n_problems, const vkwr_frag_gemm_problem* 
     if (!empty) ++bt.n;
   }
   if (bt.n == 0) return VKWR_OK;
-  const FragConfig cfg = pick_frag_config(bt);
+  const FragConfig cfg = pick_frag_config(bt, 1);
   const int bm = 32 * cfg.tm, bn = 32 * cfg.tn;
   int wgs = 0;
   for (int i = 0; i < bt.n; ++i) {
@@ -591,14 +623,20 @@ int splitk_partials(const char* fn, const vkwr_frag_gemm_problem* problem, int s
   VK_REQUIRE(workspace != nullptr && aligned16(workspace), "%s: workspace must be non-null and 16-byte aligned", fn);
   VK_REQUIRE(workspace_bytes >= need, "%s: workspace of %lld bytes, %lld needed", fn, (long long)workspace_bytes,
              (long long)need);
-  P.ncol = P.npad / kSplitTile;
-  P.nmb = (P.m + kSplitTile - 1) / kSplitTile;
+  const FragConfig cfg = pick_frag_config(bt, splits);
+  P.ncol = P.npad / (32 * cfg.tn);
+  P.nmb = (P.m + 32 * cfg.tm - 1) / (32 * cfg.tm);
+  P.ws_rows = (P.m + kSplitTile - 1) / kSplitTile * kSplitTile;
   P.xcd_map = P.ncol % 8 == 0;
   P.wg_begin = 0;
   P.ws = static_cast<float*>(workspace);
   P.ksplit = splits;
   const int wgs = (P.ncol * P.nmb * splits + 7) / 8 * 8;
-  hipLaunchKernelGGL((frag_gemm_kernel<2, 2, 8, 2, kStorePartial, false>), dim3(wgs), dim3(512), 0, stream, bt);
+  if (cfg.tm == 4) launch_partial<4, 2, 4, 2>(bt, wgs, stream);
+  else if (cfg.tm == 2) launch_partial<2, 2, 8, 2>(bt, wgs, stream);
+  else if (cfg.tn == 2) launch_partial<1, 2, 8, 2>(bt, wgs, stream);
+  else if (cfg.ks == 4) launch_partial<1, 1, 8, 4>(bt, wgs, stream);
+  else launch_partial<1, 1, 8, 2>(bt, wgs, stream);
   return VKWR_OK;
 }
 
@@ -616,7 +654,7 @@ extern "C" int vkwr_frag_gemm_splitk_f16(const vkwr_frag_gemm_problem* problem, 
   const FProb& P = bt.p[0];
   const int64_t threads = (int64_t)P.m * (P.npad / 4);
   hipLaunchKernelGGL(frag_splitk_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                     (hipStream_t)stream, P, P.nmb * kSplitTile);
+                     (hipStream_t)stream, P, P.ws_rows);
   return check_launch(fn);
 }
 
