@@ -1660,7 +1660,6 @@ __global__ __launch_bounds__((64 * rm_waves<TM, TN>())) void gemm_rm_kernel(Batc
 // activation applied and rounded to fp16 as gemm_kernel does.
 constexpr int kGvMaxM = 4;
 constexpr int kGvLdsHalfs = 32768;  // 64 KiB
-constexpr int kGvRowsNK = 16;       // [N,K]: weight rows per workgroup (4 per wave)
 constexpr int kGvColsKN = 512;      // [K,N]: columns per workgroup (a kilobyte of each k row)
 constexpr int kGvRowsKN = 8192;     // [K,N]: most k rows of one workgroup's K part
 
@@ -1678,12 +1677,21 @@ __device__ __forceinline__ void gv_stage_x(_Float16* xs, const Prob& P, int k0, 
   }
 }
 
-// [N,K] weights: a wave owns 4 rows over the whole of K; lane l reads chunks l, l + 64, ...
+// [N,K] weights: a wave owns R rows over the whole of K; lane l reads chunks l, l + 64, ...
 // of each row (a kilobyte per instruction), and the (row, m) sums are reduced across the
-// wave in a fixed order.
-template <int M, bool kMulti>
+// wave in a fixed order (the same bits for every R and U).  U chunks of a row are in flight at
+// once (gv_config chooses both).
+//
+// What bounds it: latency.  A [2048, 2048] product is 8 MB, 1.7 us of the memory's rate, in a
+// launch that cannot be shorter than ~2.5.  So the first weights are requested before the
+// activations are waited for, LDS holds no more than the activations, and a wave takes one row
+// where four left half of the CUs idle: us with weights in cache, from memory, and before (four rows):
+//   M = 1, K = N = 2048      2.7, 4.1 (3.5, 5.2)      M = 4, K = N = 2048       4.5, 5.9 (8.0, 9.4)
+//   M = 1, K 768, N 65536    17.8, 21.9 (25.8, 30.7)  M = 1, K 16384, N 4096    23.4, 26.6 (33.9, 37.2)
+//   M = 1, K 2048, N 65536   38, 43.6 (39.5, 49.5: 6.2 TB/s now)
+template <int M, int R, int U, bool kMulti>
 __global__ __launch_bounds__(256) void gemv_nk_kernel(Batch bt) {
-  __shared__ __attribute__((aligned(16))) _Float16 xs[kGvLdsHalfs];
+  extern __shared__ __attribute__((aligned(16))) _Float16 xs[];  // [m][K]
   const int t = blockIdx.x;
   int pi = 0;
   if constexpr (kMulti) {
@@ -1704,49 +1712,62 @@ __global__ __launch_bounds__(256) void gemv_nk_kernel(Batch bt) {
                  "s"(f3), "s"(f4_), "s"(f5), "s"(f6), "s"(f7), "s"(f8), "s"(f9));
   }
   const int N = P.n, K = P.k;
-  const int nr0 = (t - P.tile_begin) * kGvRowsNK;
-  gv_stage_x(xs, P, 0, K, K);
-  __syncthreads();
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int nch = K / 8;
-  float acc[4][M];
+  const int nch = K / 8, nr0 = ((t - P.tile_begin) * 4 + w) * R;
+  const _Float16* wr[R];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int r = 0; r < R; ++r) wr[r] = P.b + (int64_t)min(nr0 + r, N - 1) * K;
+  // U chunks of each of the R rows in flight per batch, every load of it issued before the first
+  // use (no branch between them); chunks past the row end are read clamped and weighted by zero.
+  hv8 wv[U][R];
+  auto request = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) wv[u][r] = *reinterpret_cast<const hv8*>(wr[r] + 8 * min(c0 + 64 * u, nch - 1));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // this thread's first activation chunk goes ahead of the weights: loads return in order
+  const int xch = P.m * nch;
+  hv8 x0 = *reinterpret_cast<const hv8*>(P.a + 8 * min((int)threadIdx.x, xch - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  request(lane);
+  for (int i = threadIdx.x; i < xch; i += 256) {  // xs is laid out as the rows of A
+    if (i >= 256) x0 = *reinterpret_cast<const hv8*>(P.a + 8 * i);
+    if (P.a_act != VKWR_GEMM_ACT_NONE) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x0[e] = (_Float16)act_in((float)x0[e], P.a_act);
+    }
+    *reinterpret_cast<hv8*>(xs + 8 * i) = x0;
+  }
+  __syncthreads();
+  float acc[R][M];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[r][m] = 0.0f;
-  const _Float16* wr[4];
+  for (int c0 = lane;;) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) wr[r] = P.b + (int64_t)min(nr0 + 4 * w + r, N - 1) * K;
-  // 4 chunks of each of the 4 rows (16 loads, 16 KiB per wave) in flight per batch; chunks
-  // past the row end are read clamped and weighted by zero.
-  constexpr int kU = 4;
-  for (int c0 = lane; c0 < nch; c0 += 64 * kU) {
-    hv8 wv[kU][4];
-#pragma unroll
-    for (int u = 0; u < kU; ++u)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        wv[u][r] = *reinterpret_cast<const hv8*>(wr[r] + 8 * min(c0 + 64 * u, nch - 1));
-    // every load of the batch is issued before the first use (no branch between them)
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int c = min(c0 + 64 * u, nch - 1);
       const bool in = c0 + 64 * u < nch;
 #pragma unroll
       for (int m = 0; m < M; ++m) {
-        hv8 xv = *reinterpret_cast<const hv8*>(xs + m * K + 8 * c);
+        hv8 xv = *reinterpret_cast<const hv8*>(xs + min(m, P.m - 1) * K + 8 * c);
         if (!in) xv = hv8{};
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < R; ++r)
 #pragma unroll
           for (int e = 0; e < 8; ++e) acc[r][m] = __builtin_fmaf((float)wv[u][r][e], (float)xv[e], acc[r][m]);
       }
     }
+    c0 += 64 * U;
+    if (c0 - lane >= nch) break;
+    request(c0);
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int n = nr0 + 4 * w + r;
+  for (int r = 0; r < R; ++r) {
+    const int n = nr0 + r;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       const float s = wave_sum(acc[r][m]);
@@ -1894,6 +1915,7 @@ struct Config {
   bool kn = false;  // ... with [K,N] weights
   int gv = 0;       // gemv_{nk,kn}_kernel<gv> (M <= gv <= 4), 0: not this path
   int mid = 0;      // gemm_mid_kernel (bm x bn tiles, K in `mid` parts), 0: not this path
+  int gv_u = 0;     // gemv_nk_kernel: chunks of a row in flight (bn / 4 rows per wave)
 };
 
 // Tile shape from the largest M of the batch (all problems of one launch share it).
@@ -2004,7 +2026,21 @@ bool gv_config(const Batch& bt, int max_m, Config& cfg) {
     if (!P.b_kn && (int64_t)max_m * P.k > kGvLdsHalfs) return false;
   }
   if (kn < 0) return false;
-  cfg = Config{1, kn ? kGvColsKN : kGvRowsNK, false, false, kn == 1, max_m <= 2 ? max_m : 4};
+  cfg = Config{1, kGvColsKN, false, false, kn == 1, max_m <= 2 ? max_m : 4};
+  if (kn) return true;
+  int64_t rows = 0;
+  int max_k = 0;
+  for (int i = 0; i < bt.n; ++i)
+    if (bt.p[i].m > 0 && bt.p[i].n > 0) rows += bt.p[i].n, max_k = std::max(max_k, bt.p[i].k);
+  // K <= 512 (the low-rank outputs): one chunk per lane, two rows per wave where one would make many
+  // short-lived workgroups (four of N 2048, M = 1: 3.3 us, one row 3.6, four rows and chunks 5.1; four of
+  // N 4096: 4.2, 5.4, 8.5; M = 2, four of N 2048: 4.6, 4.3).  Longer K: one row per wave; with
+  // three or four activation rows, which every wave reads from LDS for each weight row, two once
+  // the weights come to 16384 rows (M = 4, K 2048, N 32768, weights from memory: 38.3, one row 39.6).
+  const bool short_k = max_k <= 512;
+  const bool two = short_k ? rows > 4096 * cfg.gv : cfg.gv == 4 && rows >= 16384;
+  cfg.gv_u = short_k ? 1 : 4;
+  cfg.bn = two ? 8 : 4;
   return true;
 }
 
@@ -2530,6 +2566,26 @@ static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
 
+template <int M, bool kMulti>
+void gv_nk_launch(const Config& cfg, const Batch& bt, int wgs, hipStream_t s) {
+  int64_t lds = 0;
+  for (int i = 0; i < bt.n; ++i)
+    if (bt.p[i].n > 0) lds = std::max(lds, (int64_t)bt.p[i].m * bt.p[i].k * 2);
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(wgs), dim3(256), (size_t)lds, s, bt); };
+  if (cfg.gv_u == 1) {
+    if (cfg.bn == 8) go(gemv_nk_kernel<M, 2, 1, kMulti>);
+    else go(gemv_nk_kernel<M, 1, 1, kMulti>);
+    return;
+  }
+  if constexpr (M == kGvMaxM) {
+    if (cfg.bn == 8) {
+      go(gemv_nk_kernel<M, 2, 4, kMulti>);
+      return;
+    }
+  }
+  go(gemv_nk_kernel<M, 1, 4, kMulti>);
+}
+
 template <int BM, int BN, int NBUF>
 void mid_launch_tile(bool kn, bool act, const Batch& bt, int wgs, hipStream_t s) {
   auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(wgs), dim3(256), 0, s, bt, wgs); };
@@ -2589,9 +2645,9 @@ int gemm_run(const char* fn, Batch& bt, const Config& cfg, BigPlan& pl, void* wo
     } else {
       auto go_gv = [&](auto multi) {
         constexpr bool kM = decltype(multi)::value;
-        if (cfg.gv == 1) hipLaunchKernelGGL((gemv_nk_kernel<1, kM>), dim3(wgs), dim3(256), 0, s, bt);
-        else if (cfg.gv == 2) hipLaunchKernelGGL((gemv_nk_kernel<2, kM>), dim3(wgs), dim3(256), 0, s, bt);
-        else hipLaunchKernelGGL((gemv_nk_kernel<4, kM>), dim3(wgs), dim3(256), 0, s, bt);
+        if (cfg.gv == 1) gv_nk_launch<1, kM>(cfg, bt, wgs, s);
+        else if (cfg.gv == 2) gv_nk_launch<2, kM>(cfg, bt, wgs, s);
+        else gv_nk_launch<4, kM>(cfg, bt, wgs, s);
       };
       if (bt.n > 1) go_gv(std::true_type{});
       else go_gv(std::false_type{});
