@@ -77,7 +77,8 @@ VKWR_EXPORT int vkwr_wkv7_fp32_forward_slots(int B, int T, int C, int H, float* 
  * vkwr_wkv7_fp32_forward_slots (slots given: state is the pool) with device scratch: where
  * the batch has too few (sequence, head) chains to fill the GPU, a long prefill is cut into
  * segments along T that run side by side and are joined through the scratch.  Same values to
- * fp32 rounding.  workspace: vkwr_wkv7_fp32_prefill_workspace_bytes(B, T, H) bytes, 16-byte
+ * fp32 rounding, for any a and b: a chain whose transitions grow past 2^60 inside a segment, or
+ * that meets a NaN, is run token by token (finite where the recurrence is).  workspace: vkwr_wkv7_fp32_prefill_workspace_bytes(B, T, H) bytes, 16-byte
  * aligned; with less, or NULL, the call runs without segments, as the entry points above.
  * ..._workspace_max(rows, H): enough for every B, T with B * T <= rows.
  * Replaces the device work of vkwr_v1_wkv::wkv_forward_fp32 (csrc/v1/wkv/torch_bindings.cpp:179-188). */

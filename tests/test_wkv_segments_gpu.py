@@ -124,3 +124,52 @@ def test_segments_out_of_range_slot_and_short_scratch(gpu):
     err = (y.float() - plain.float()).abs()
     ulp = torch.exp2(torch.floor(torch.log2(plain.float().abs().clamp_min(2.0 ** -14))) - 10)
     assert bool((err <= ulp + 2e-5 * plain.float().abs().max()).all()) and (pool - plain_pool).abs().max().item() <= 2e-5 * plain_pool.abs().max().item()
+
+
+@pytest.mark.parametrize("B,T,H", [(1, 1500, 32), (2, 700, 5), (1, 100003, 2)])
+@pytest.mark.parametrize("what", ["overflow", "nan"])
+def test_segments_where_the_transitions_overflow(gpu, B, T, H, what):
+    """The op takes any a and b.  In one head they make a mode grow by d + 7 a token that the state
+    never holds (column 0: zero at the start, k_0 = 0), so the chain stays finite while the product of a
+    segment's transitions passes fp32's largest value after ~45 tokens; or one v is NaN, which reaches
+    its own value row from its token on and nothing else.  Such a chain against the oracle (fp32 sums
+    in another order: the state contract's 2e-5 of the largest value, then y's rounding); the other
+    heads give what they give beside ordinary ones."""
+    C, hz = H * 64, H - 1
+    ins = make_wkv_inputs(B, T, H, seed=T + B, dist="realistic")
+    clean = [x.copy() for x in ins]
+    r, w, k, v, a, b = (x.reshape(B, T, H, 64) for x in ins)
+    state_np = make_state(B, H, seed=3)
+    if what == "overflow":
+        a[:, :, hz], b[:, :, hz], k[:, :, hz, 0] = 0, 0, 0
+        a[:, :, hz, 0], b[:, :, hz, 0] = 1, 7
+        state_np[:, hz] = 0
+    else:
+        v[0, T // 3, hz, 7] = np.nan
+    need = capi._LIB.vkwr_wkv7_fp32_prefill_workspace_bytes(B, T, H)
+    assert need > 0
+    slots = torch.arange(B, dtype=torch.int32, device=gpu)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=gpu)
+
+    def run(arrays):
+        pool = torch.from_numpy(state_np.copy()).to(gpu)
+        y = torch.empty(B, T, C, dtype=torch.float16, device=gpu)
+        capi.wkv_slots(B, T, C, H, pool, slots, *_dev(arrays, gpu), y, workspace=ws)
+        torch.cuda.synchronize()
+        return y.view(B, T, H, 64).cpu(), pool.cpu()
+
+    y, state = run(ins)
+    s_ref = np.ascontiguousarray(state_np[:, hz:])
+    one = [np.ascontiguousarray(x.reshape(B, T, H, 64)[:, :, hz]) for x in ins]
+    y_ref = orc.wkv_fp32(B, T, 64, 1, s_ref, *one).astype(np.float64)
+    got, s_got = y[:, :, hz].numpy().astype(np.float64), state[:, hz].numpy()
+    s_ref = s_ref[:, 0]
+    assert np.isnan(y_ref).any() == (what == "nan")
+    assert np.array_equal(np.isnan(got), np.isnan(y_ref)) and np.array_equal(np.isnan(s_got), np.isnan(s_ref))
+    top = np.nanmax(np.abs(s_ref))
+    assert np.nanmax(np.abs(s_got - s_ref)) <= 2e-5 * top
+    ulp = np.exp2(np.floor(np.log2(np.maximum(np.abs(np.nan_to_num(y_ref)), 2.0 ** -14))) - 10)
+    assert (np.nan_to_num(np.abs(got - y_ref)) <= ulp + 2e-5 * np.nanmax(np.abs(y_ref))).all()
+    if H > 1:
+        y2, state2 = run(clean)
+        assert torch.equal(y[:, :, :hz], y2[:, :, :hz]) and torch.equal(state[:, :hz], state2[:, :hz])

@@ -841,14 +841,30 @@ struct ChunkLds {
 // sums of the one-chain form: against 64 bits the state is off by 3.4e-7 (one chain 2.7e-7; 3.8e-7
 // with Λ formed as a product), y by its fp16 rounding.  T is taken in blocks of `len` tokens so
 // that the scratch stays bounded.  What bounds it: 3.4 us per chunk of a segment (the state waves'
-// products) and ~26 us of pipeline fill and launches; 32 chains, T = 1500: 220 -> 75 us.
+// products) and ~26 us of pipeline fill and launches; 32 chains, T = 1500: 217 -> 77 us.
+//
+// M and q carry every mode of the transitions, also those that the state never excites: for the
+// model's a = -kk, b = a kk they contract, but the call takes any a and b, and where M overflows
+// under a state of zeros 0 * inf would make NaN of rows that one chain keeps finite.  So every M, N,
+// q, y0 and S_start is held against kSegMax, below which no sum of steps 2 and 3 can overflow; a
+// chain with a value beyond it, or a NaN, is run token by token in step 2 instead, from the state
+// that it still has (1.25 us a token: for such inputs only).  Looking costs every call 1 - 2 us (T =
+// 1500: 75.4 -> 76.8); a further launch of the one-chain kernel for such chains would cost 3.
 struct SegArgs {
   int P, cps;    // segments, chunks per segment
   int t0, len;   // tokens of this block
   float *m, *n;  // [chains][P][64][64]
   float* start;  // [chains][P][64][64] S_start of every segment
+  int* wide;     // [chains][P][4] a state wave saw a value beyond kSegMax
+  int* done;     // [chains] step 2 ran the chain token by token
   float *q, *y0; // [B][len][C]
 };
+
+// The largest magnitude as bits: as unsigned numbers those of NaN and Inf are above every finite one's.
+__device__ __forceinline__ uint32_t seg_top(uint32_t top, float x) {
+  return max(top, __builtin_bit_cast(uint32_t, x) & 0x7fffffffu);
+}
+constexpr uint32_t kSegMax = (127 + 60) << 23;  // 2^60: 64 products of two such values stay below 2^127
 
 // Eight waves in two roles, two per SIMD (waves w and w + 4 share SIMD w), so that each
 // SIMD interleaves two independent instruction streams.  State waves 0-3 own the state rows
@@ -860,7 +876,7 @@ struct SegArgs {
 // (116 / 112 / 96 / 96 products per SIMD and chunk).  One barrier per chunk.  The LDS
 // pipeline (four hat buffers, three matrix buffers) takes 144 KiB: one workgroup per CU.
 //
-// kSeg: the first of the three launches of a prefill cut into segments (SegArgs below).  The
+// kSeg: the first of the three launches of a prefill cut into segments (SegArgs above).  The
 // workgroup takes one segment of the (sequence, head) from an unknown start state: its state
 // waves run the same chunk products on two states, M from the identity without the v k^T
 // updates, and N from zero, and store for every token M's output (the query that the start
@@ -890,6 +906,7 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra, SegAr
   // X^T tile q (j = 16 q .. 16 q + 15): register r holds X^T[16 q + 4 g + r][iw] = S[iw][16 q + 4 g + r]
   fq4 st[4];
   fq4 sm[4];  // (kSeg) the same of M; st is N
+  uint32_t top = 0;
   if (kSeg) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -1206,6 +1223,8 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra, SegAr
             sg.y0[at + (size_t)r * C] = y1[r];
             sg.q[at + (size_t)r * C] = ym1[r];
           }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) top = seg_top(seg_top(top, y1[r]), ym1[r]);
       } else {
         // y rows t = 4 g + r of this wave's 16 value columns
         _Float16 yh[4];
@@ -1236,7 +1255,13 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra, SegAr
     if constexpr (kSeg) {
       float* const Mo = sg.m + (size_t)blockIdx.x * kHead * kHead;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) *reinterpret_cast<fq4*>(Mo + iw * kHead + 16 * q + 4 * g) = sm[q];
+      for (int q = 0; q < 4; ++q) {
+        *reinterpret_cast<fq4*>(Mo + iw * kHead + 16 * q + 4 * g) = sm[q];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) top = seg_top(seg_top(top, st[q][r]), sm[q][r]);
+      }
+      const bool wide = __ballot(top > kSegMax) != 0;
+      if (lane == 0) sg.wide[4 * blockIdx.x + w] = wide;
     }
   } else {
     // The matrix waves' work is dependent chains (W^T's powers, LDS round trips, the Λ scans);
@@ -1259,12 +1284,62 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra, SegAr
   }
 }
 
+// `len` tokens of one chain, one after the other, by 1024 threads: thread tid holds row tid / 16, columns
+// 4 (tid % 16) .. + 3 of the state S (64 x 64).  The next token's vectors are requested a token ahead.
+__device__ __forceinline__ void chain_tokens(const Fp32Args& p, float* S, size_t tok0, int len) {
+  const int tid = threadIdx.x, i = tid >> 4, j = 4 * (tid & 15);
+  struct Tok {
+    _Float16 r[4], w[4], k[4], a[4], b[4], v;
+  };
+  auto fetch = [&](int t) __attribute__((always_inline)) {
+    const size_t at = tok0 + (size_t)min(t, len - 1) * p.C;
+    Tok x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x.r[e] = p.r[at + j + e], x.w[e] = p.w[at + j + e], x.k[e] = p.k[at + j + e];
+      x.a[e] = p.a[at + j + e], x.b[e] = p.b[at + j + e];
+    }
+    x.v = p.v[at + i];
+    return x;
+  };
+  auto sum16 = [](float x) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) x += __shfl_xor(x, o, 16);
+    return x;
+  };
+  float s[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) s[e] = S[i * kHead + j + e];
+  Tok nx = fetch(0);
+  for (int t = 0; t < len; ++t) {
+    const Tok x = nx;
+    nx = fetch(t + 1);
+    float sa = 0.0f, y = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sa = __builtin_fmaf(s[e], (float)x.a[e], sa);
+    sa = sum16(sa);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float z = s[e] * __builtin_amdgcn_exp2f(log2_decay_fast((float)x.w[e]));
+      z = __builtin_fmaf(sa, (float)x.b[e], z);
+      s[e] = __builtin_fmaf((float)x.k[e], (float)x.v, z);
+      y = __builtin_fmaf(s[e], (float)x.r[e], y);
+    }
+    y = sum16(y);
+    __syncthreads();  // every thread has read the token's vectors: y may be one of them
+    if ((tid & 15) == 0) p.y[tok0 + (size_t)t * p.C + i] = (_Float16)y;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) S[i * kHead + j + e] = s[e];
+}
+
 // Step 2: one workgroup of 16 waves per chain, wave (ri, cj) the 16 x 16 tile of S = S M_p + N_p at
 // rows 16 ri, columns 16 cj.  S goes through LDS as the next product's A operand; the next
 // segment's M and N tiles are requested before the current products.
 template <bool kSlots>
 __global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(Fp32Args p, SegArgs sg) {
   __shared__ __attribute__((aligned(16))) float s[kHead][kHP];
+  __shared__ int apart;  // some value is beyond kSegMax
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 15, g = lane >> 4, ri = w >> 2, cj = w & 3;
   const int bh = blockIdx.x, bi = bh / p.H, h = bh - bi * p.H;
@@ -1274,6 +1349,7 @@ __global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(Fp32Args p, SegArgs
   // B operand of k step (q, s2): M[16 q + 4 g + s2][16 cj + li]
   float mb[2][16];
   fq4 nt[2];
+  uint32_t top = 0;
   auto load = [&](int seg, int set) __attribute__((always_inline)) {
     const float* M = sg.m + base + (size_t)seg * kHead * kHead + 16 * cj + li;
     const float* N = sg.n + base + (size_t)seg * kHead * kHead + (16 * ri + 4 * g) * kHead + 16 * cj + li;
@@ -1285,8 +1361,10 @@ __global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(Fp32Args p, SegArgs
   auto step = [&](int seg, int set) __attribute__((always_inline)) {
     if (seg + 1 < sg.P) load(seg + 1, set ^ 1);
     // S_start of this segment: thread -> 4 consecutive floats
-    *reinterpret_cast<fq4*>(sg.start + base + (size_t)seg * kHead * kHead + tid * 4) =
-        *reinterpret_cast<const fq4*>(&s[tid >> 4][4 * (tid & 15)]);
+    const fq4 here = *reinterpret_cast<const fq4*>(&s[tid >> 4][4 * (tid & 15)]);
+    *reinterpret_cast<fq4*>(sg.start + base + (size_t)seg * kHead * kHead + tid * 4) = here;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) top = seg_top(top, here[r]);
     fq4 a[4], acc = nt[set];
 #pragma unroll
     for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const fq4*>(&s[16 * ri + li][16 * q + 4 * g]);
@@ -1300,13 +1378,24 @@ __global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(Fp32Args p, SegArgs
     __syncthreads();
   };
   *reinterpret_cast<fq4*>(&s[tid >> 4][4 * (tid & 15)]) = *reinterpret_cast<const fq4*>(S + tid * 4);
+  if (tid == 0) apart = 0;
   load(0, 0);
+  const int wide = sg.wide[4 * bh * sg.P + min(tid, 4 * sg.P - 1)];  // (P <= 256; no branch, no wait here)
   __syncthreads();
   for (int seg = 0; seg < sg.P; seg += 2) {
     step(seg, 0);
     if (seg + 1 < sg.P) step(seg + 1, 1);
   }
-  *reinterpret_cast<fq4*>(S + tid * 4) = *reinterpret_cast<const fq4*>(&s[tid >> 4][4 * (tid & 15)]);
+  const fq4 end = *reinterpret_cast<const fq4*>(&s[tid >> 4][4 * (tid & 15)]);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) top = seg_top(top, end[r]);
+  if (__ballot(top > kSegMax || wide) != 0 && lane == 0) apart = 1;
+  __syncthreads();
+  if (tid == 0) sg.done[bh] = apart;
+  if (apart)
+    chain_tokens(p, S, ((size_t)bi * p.T + sg.t0) * p.C + (size_t)h * kHead, sg.len);
+  else
+    *reinterpret_cast<fq4*>(S + tid * 4) = end;
 }
 
 // Step 3: one workgroup per (chain, segment), wave w its chunks w, w + 4, ...: 16 tokens x 64
@@ -1322,6 +1411,7 @@ __global__ __launch_bounds__(256) void wkv_seg_out_kernel(Fp32Args p, SegArgs sg
     for (int idx = tid; idx < T * kHead; idx += 256) y[(size_t)(idx / kHead) * C + idx % kHead] = (_Float16)__builtin_nanf("");
     return;
   }
+  const int done = sg.done[bh];  // (looked at only by the stores: S and q are not held up behind it)
   const float* S = sg.start + (size_t)blockIdx.x * kHead * kHead;
   const size_t tok = ((size_t)bi * sg.len + s0) * C + (size_t)h * kHead;
   fq4 sb[4][4];  // B operand of output tile c: S_start[16 c + li][16 q + 4 g ..]
@@ -1348,7 +1438,7 @@ __global__ __launch_bounds__(256) void wkv_seg_out_kernel(Fp32Args p, SegArgs sg
         for (int c = 0; c < 4; ++c) acc[c] = mfma4(a[q][s2], sb[c][q][s2], acc[c]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      if (c0 + 4 * g + r >= T) continue;
+      if (done || c0 + 4 * g + r >= T) continue;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         float v = acc[c][r];
@@ -1377,12 +1467,12 @@ SegPlan seg_plan(int B, int T, int H) {
   const int len = ((T + blocks - 1) / blocks + kCL - 1) / kCL * kCL;
   const int nchunk = (std::min(len, T) + kCL - 1) / kCL;
   // Time model (us), both sides measured: one chain per workgroup 9.3 + 2.24 per chunk (T = 300: 52,
-  // T = 1500: 220); P segments 26 + 3.4 per chunk of a segment + 0.9 P (32 chains, T = 300, P = 6: 42;
-  // T = 1500, P = 8: 78; T = 4096: 587 -> 151; 128 chains, T = 1024, P = 2: 159 -> 145; below
+  // T = 1500: 217); P segments 26 + 3.4 per chunk of a segment + 0.9 P (32 chains, T = 300, P = 6: 42;
+  // T = 1500, P = 8: 77; T = 4096: 580 -> 150; 128 chains, T = 1024, P = 2: 151 -> 139; below
   // ~12 chunks the two extra launches cost more than they save: T = 128 27 against 32).
   double best = 0.92 * (9.3 + 2.24 * nchunk);
   SegPlan plan = one;
-  for (int P = 2; P <= G / chains && 2 * P <= nchunk; ++P) {
+  for (int P = 2; P <= std::min<int64_t>(G / chains, 256) && 2 * P <= nchunk; ++P) {
     const int cps = (nchunk + P - 1) / P;
     if ((nchunk + cps - 1) / cps != P) continue;
     const double t = 26 + 3.4 * cps + 0.9 * P;
@@ -1394,10 +1484,13 @@ SegPlan seg_plan(int B, int T, int H) {
   return plan;
 }
 
+// wide and done, in whole cache lines: with q's rows off by 112 bytes 12 chains of 700 tokens took 3 us longer
+int64_t seg_marks(int64_t chains, int64_t P) { return (4 * chains * P + chains + 63) / 64 * 64; }
+
 int64_t seg_bytes(const SegPlan& s, int B, int H) {
   if (s.P == 1) return 0;
   const int64_t chains = (int64_t)B * H;
-  return (chains * s.P * 3 * kHead * kHead + 2 * chains * s.len * kHead) * 4;
+  return (chains * s.P * 3 * kHead * kHead + seg_marks(chains, s.P) + 2 * chains * s.len * kHead) * 4;
 }
 
 bool rows_vec_ok(const Fp32Args& p) {
@@ -1430,10 +1523,12 @@ void launch_fp32(const Fp32Args& p, int B, hipStream_t stream, bool rows, void* 
       }
       const int64_t mat = (int64_t)B * p.H * s.P * kHead * kHead;
       float* f = reinterpret_cast<float*>(ws);
+      int* const marks = reinterpret_cast<int*>(f + 3 * mat);
+      float* const rows = f + 3 * mat + seg_marks((int64_t)B * p.H, s.P);
       for (int t0 = 0; t0 < p.T; t0 += s.len) {
         const int len = std::min(s.len, p.T - t0), nchunk = (len + kCL - 1) / kCL;
-        SegArgs sg{(nchunk + s.cps - 1) / s.cps, s.cps, t0, len, f, f + mat, f + 2 * mat, f + 3 * mat,
-                   f + 3 * mat + (int64_t)B * len * p.C};
+        SegArgs sg{(nchunk + s.cps - 1) / s.cps, s.cps, t0, len, f, f + mat, f + 2 * mat,
+                   marks, marks + (int64_t)4 * B * p.H * s.P, rows, rows + (int64_t)B * len * p.C};
         const dim3 grid(B * p.H * sg.P);
         hipLaunchKernelGGL((wkv7_fp32_chunk_kernel<kSlots, true>), grid, dim3(512), 0, stream, ra, sg);
         hipLaunchKernelGGL(wkv_seg_chain_kernel<kSlots>, dim3(B * p.H), dim3(1024), 0, stream, p, sg);
@@ -2207,7 +2302,7 @@ extern "C" int64_t vkwr_wkv7_fp32_prefill_workspace_max(int64_t rows, int H) {
   // the matrices of at most a segment per CU, and the rows of one block (a block's length is rounded
   // up to whole chunks, of at most half a chain per CU)
   const int64_t G = device_cus();
-  return (G * 3 * kHead * kHead) * 4 + std::min(rows * H * kHead * 8, kSegMaxBytes + G / 2 * kCL * kHead * 8);
+  return (G * 3 * kHead * kHead + seg_marks(G / 2, 2)) * 4 + std::min(rows * H * kHead * 8, kSegMaxBytes + G / 2 * kCL * kHead * 8);
 }
 
 extern "C" int vkwr_wkv7_fp32_prefill(int B, int T, int C, int H, float* state, int n_slots, const int32_t* slots,
