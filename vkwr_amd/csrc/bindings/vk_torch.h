@@ -9,8 +9,10 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/Exception.h>
 #include <torch/library.h>
 
+#include <exception>
 #include <vector>
 
 #include "vkwr_amd.h"
@@ -68,16 +70,31 @@ inline T* ptr(const at::Tensor& x) {
   return reinterpret_cast<T*>(x.data_ptr());
 }
 
+// Device scratch from torch's caching allocator, or an undefined tensor where it has no memory left (then
+// *oom, if given, holds its exception): for calls that scratch makes faster but that run without.
+inline at::Tensor try_scratch(int64_t bytes, const at::Tensor& like, std::exception_ptr* oom = nullptr) {
+  if (bytes <= 0) return {};
+  try {
+    return at::empty({bytes}, like.options().dtype(at::kByte));
+  } catch (const c10::OutOfMemoryError&) {
+    if (oom) *oom = std::current_exception();
+    return {};
+  }
+}
+
 // Runs a batch of GEMMs (include/vkwr_amd.h vkwr_gemm_f16) on the current
 // stream, with the K-split workspace taken from torch's caching allocator.
+// Without memory for it a batch that can runs in fewer K parts; the others throw
+// the allocator's error.
 inline void run_gemm(std::vector<vkwr_gemm_problem>& probs, const at::Tensor& like, const char* what) {
   const int64_t ws = vkwr_gemm_f16_workspace_bytes((int)probs.size(), probs.data());
   check_status(ws < 0 ? VKWR_ERR_INVALID : VKWR_OK, what);
-  at::Tensor w;
-  if (ws > 0) w = at::empty({ws}, like.options().dtype(at::kByte));
-  check_status(vkwr_gemm_f16((int)probs.size(), probs.data(), ws > 0 ? w.data_ptr() : nullptr, ws,
-                             stream()),
-               what);
+  std::exception_ptr oom;
+  const at::Tensor w = try_scratch(ws, like, &oom);
+  const int st = vkwr_gemm_f16((int)probs.size(), probs.data(), w.defined() ? w.data_ptr() : nullptr,
+                               w.defined() ? ws : 0, stream());
+  if (st != VKWR_OK && oom) std::rethrow_exception(oom);
+  check_status(st, what);
 }
 
 inline vkwr_gemm_problem gemm_problem(const at::Tensor& a, const at::Tensor& b, at::Tensor& c,

@@ -135,17 +135,17 @@ void check_wkv_fp32_io(int64_t B, int64_t T, int64_t C, int64_t H, const at::Ten
   check_fits_int(C, "C");
 }
 
-// Mode 0 / slot pool with the scratch of a segmented prefill from torch's caching allocator.
+// Mode 0 / slot pool with the scratch of a segmented prefill from torch's caching allocator (up to
+// ~110 MB; a captured call keeps it in its graph's pool), or in one chain each where it has none.
 int wkv_prefill(int64_t B, int64_t T, int64_t C, int64_t H, at::Tensor& state, int64_t n_slots, const int32_t* slots,
                 const at::Tensor& r, const at::Tensor& w, const at::Tensor& k, const at::Tensor& v,
                 const at::Tensor& a, const at::Tensor& b, at::Tensor& y) {
   const int64_t bytes = vkwr_wkv7_fp32_prefill_workspace_bytes((int)B, (int)T, (int)H);
-  at::Tensor ws;
-  if (bytes > 0) ws = at::empty({bytes}, r.options().dtype(at::kByte));
+  const at::Tensor ws = try_scratch(bytes, r);
   return vkwr_wkv7_fp32_prefill((int)B, (int)T, (int)C, (int)H, ptr<float>(state), (int)n_slots, slots,
                                 ptr<uint16_t>(r), ptr<uint16_t>(w), ptr<uint16_t>(k), ptr<uint16_t>(v),
                                 ptr<uint16_t>(a), ptr<uint16_t>(b), ptr<uint16_t>(y),
-                                bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream());
+                                ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? bytes : 0, stream());
 }
 
 void wkv_fp32_mode(int64_t B, int64_t T, int64_t C, int64_t H, at::Tensor& state,
