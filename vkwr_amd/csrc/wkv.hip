@@ -1457,30 +1457,39 @@ struct SegPlan {
 
 constexpr int64_t kSegMaxBytes = (int64_t)96 << 20;  // of q and y0
 
-SegPlan seg_plan(int B, int T, int H) {
-  SegPlan one{1, 0, T};
-  const int64_t chains = (int64_t)B * H;
-  const int G = device_cus();
-  if (T < kChunkMinT || 2 * chains > G) return one;
-  const int64_t most = kSegMaxBytes / (chains * kHead * 8);  // tokens of a block
-  const int blocks = (int)((T + most - 1) / most);
-  const int len = ((T + blocks - 1) / blocks + kCL - 1) / kCL * kCL;
-  const int nchunk = (std::min(len, T) + kCL - 1) / kCL;
+// P segments of cps chunks for a block of nchunk chunks, or P = 1 where one chain each takes no longer.
+SegPlan seg_split(int64_t chains, int nchunk) {
   // Time model (us), both sides measured: one chain per workgroup 9.3 + 2.24 per chunk (T = 300: 52,
   // T = 1500: 217); P segments 26 + 3.4 per chunk of a segment + 0.9 P (32 chains, T = 300, P = 6: 42;
   // T = 1500, P = 8: 77; T = 4096: 580 -> 150; 128 chains, T = 1024, P = 2: 151 -> 139; below
   // ~12 chunks the two extra launches cost more than they save: T = 128 27 against 32).
   double best = 0.92 * (9.3 + 2.24 * nchunk);
-  SegPlan plan = one;
-  for (int P = 2; P <= std::min<int64_t>(G / chains, 256) && 2 * P <= nchunk; ++P) {
+  SegPlan plan{1, 0, 0};
+  const int64_t most = std::min<int64_t>(device_cus() / chains, 256);
+  for (int P = 2; P <= most && 2 * P <= nchunk; ++P) {
     const int cps = (nchunk + P - 1) / P;
     if ((nchunk + cps - 1) / cps != P) continue;
     const double t = 26 + 3.4 * cps + 0.9 * P;
     if (t < best) {
       best = t;
-      plan = SegPlan{P, cps, std::min(len, T)};
+      plan = SegPlan{P, cps, 0};
     }
   }
+  return plan;
+}
+
+bool seg_few(int64_t chains) { return 2 * chains <= device_cus(); }
+
+int64_t seg_block(int64_t chains) { return kSegMaxBytes / (chains * kHead * 8); }  // most tokens of a block
+
+SegPlan seg_plan(int B, int T, int H) {
+  const int64_t chains = (int64_t)B * H;
+  if (T < kChunkMinT || !seg_few(chains)) return SegPlan{1, 0, T};
+  const int64_t most = seg_block(chains);
+  const int blocks = (int)((T + most - 1) / most);
+  const int len = ((T + blocks - 1) / blocks + kCL - 1) / kCL * kCL;
+  SegPlan plan = seg_split(chains, (std::min(len, T) + kCL - 1) / kCL);
+  plan.len = plan.P == 1 ? T : std::min(len, T);
   return plan;
 }
 
@@ -2299,10 +2308,16 @@ extern "C" int64_t vkwr_wkv7_fp32_prefill_workspace_bytes(int B, int T, int H) {
 
 extern "C" int64_t vkwr_wkv7_fp32_prefill_workspace_max(int64_t rows, int H) {
   if (rows <= 0 || H <= 0) return 0;
-  // the matrices of at most a segment per CU, and the rows of one block (a block's length is rounded
-  // up to whole chunks, of at most half a chain per CU)
-  const int64_t G = device_cus();
-  return (G * 3 * kHead * kHead + seg_marks(G / 2, 2)) * 4 + std::min(rows * H * kHead * 8, kSegMaxBytes + G / 2 * kCL * kHead * 8);
+  int64_t most = 0;  // 0 where no B, T of that many rows is cut into segments
+  for (int B = 1; seg_few((int64_t)B * H) && B * kChunkMinT <= rows; ++B) {
+    const int64_t chains = (int64_t)B * H, T = std::min(rows / B, (seg_block(chains) + kCL - 1) / kCL * kCL);
+    for (int n = 1; n <= (T + kCL - 1) / kCL; ++n) {  // a block of n chunks
+      SegPlan s = seg_split(chains, n);
+      s.len = (int)std::min<int64_t>(T, n * kCL);
+      most = std::max(most, seg_bytes(s, B, H));
+    }
+  }
+  return most;
 }
 
 extern "C" int vkwr_wkv7_fp32_prefill(int B, int T, int C, int H, float* state, int n_slots, const int32_t* slots,
