@@ -82,3 +82,23 @@ def test_planner_batch_with_one_empty_problem():
     alone = capi.gemm_workspace_bytes([_problem(8, 2048, 2048)])
     assert capi.gemm_workspace_bytes([_problem(0, 2048, 2048), _problem(8, 2048, 2048)]) == alone
     assert alone > 0  # 8 rows x 16 tiles leave the CUs idle: K is split
+
+
+@pytest.mark.parametrize("C", [768, 1024, 1536, 2048, 2560, 3072, 4096])
+def test_value_parts_of_every_batch(C):
+    """K parts of the decode engine's FFN value GEMM: whole steps of 256, at least as many as 64 x 64
+    tiles alone get, and a number that the next LayerNorm adds where theirs is one."""
+    cfg = types.SimpleNamespace(n_embd=C, dim_ffn=4 * C)
+
+    def parts(B):
+        return DecodeEngine._value_splits(types.SimpleNamespace(cfg=cfg), B)
+
+    for B in range(1, 513):
+        n = min(16, max(1, 256 // (-(-B // 64) * (C // 64))))
+        while n > 1 and 4 * C % (256 * n):
+            n //= 2  # n: the parts that 64 x 64 tiles alone get
+        got = parts(B)
+        assert 4 * C % (256 * got) == 0 and got >= n, (B, got, n)
+        assert n not in (2, 4, 8) or got in (2, 4, 8), (B, got, n)
+    assert {2048: [8, 8, 4, 4, 4, 2], 2560: [1, 1, 1, 2, 2, 2], 4096: [4, 4, 4, 2, 2, 1],
+            1536: [2, 2, 2, 3, 3, 2]}.get(C) in (None, [parts(B) for B in (8, 64, 128, 160, 192, 300)])

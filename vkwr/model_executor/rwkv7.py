@@ -165,6 +165,7 @@ class RWKV7State:
         return cfg.n_layer * (2 * cfg.n_head * HEAD * HEAD * 4 + 2 * 2 * cfg.n_embd * 2)
 
 
+LN_PARTS = (2, 4, 8)  # numbers of K parts that add_layer_norm_mix_parts takes
 FRAG_WEIGHTS = ("Wr", "Wk", "Wv", "Wo", "w1", "w2", "a1", "a2", "g1", "g2", "v1", "v2", "key", "value")
 
 
@@ -234,15 +235,25 @@ class DecodeEngine:
 
     def _value_splits(self, B):
         """K parts of the FFN value GEMM at batch B: enough 64x64-tile parts (128x64 where 64x64 tiles
-        alone come to 96 or more) to give the 256 CUs one workgroup each, each part at least 256 deep
-        in K.  C = 2048, B = 160: 4 parts of 128x64 18.8 us, 2 of 64x64 20.3; C = 4096, B = 128: 36.8, 42.5."""
+        alone come to 96 or more and the larger ones leave more parts) to give the 256 CUs one workgroup
+        each, each part at least 256 deep in K.  C = 2048, B = 160: 4 parts of 128x64 18.8 us, 2 of 64x64
+        20.3; C = 4096, B = 128: 36.8, 42.5.  A number of parts that the next LayerNorm adds is not given up
+        for another: six layers at C = 1536, B = 300 take 748 us with 2 parts, 772 with 3 (C = 2560, B = 160,
+        where 128x64 tiles leave one part: 885 us with 2, 918 with 1)."""
         C, F = self.cfg.n_embd, self.cfg.dim_ffn
-        tiles = -(-B // 64) * (capi.frag_pad(C) // 64)
+
+        def parts(rows):
+            tiles = -(-B // rows) * (capi.frag_pad(C) // 64)
+            n = max(1, min(16, 256 // max(tiles, 1)))
+            while n > 1 and capi.frag_pad(F) % (256 * n):
+                n //= 2
+            return tiles, n
+
+        tiles, splits = parts(64)
         if tiles >= 96:
-            tiles = -(-B // 128) * (capi.frag_pad(C) // 64)
-        splits = max(1, min(16, 256 // max(tiles, 1)))
-        while splits > 1 and capi.frag_pad(F) % (256 * splits):
-            splits //= 2
+            _, wide = parts(128)
+            if wide > splits and (wide in LN_PARTS or splits not in LN_PARTS):
+                splits = wide
         return splits
 
     def _step_frag(self, state, tokens, slots):
@@ -252,8 +263,8 @@ class DecodeEngine:
         fp = capi.frag_problem
         x, res_in, parts = None, None, 0
         splits = self._value_splits(B)
-        # FFN value K parts reduced inside the next layer's LayerNorm (2, 4 or 8 parts)
-        parts_ok = splits in (2, 4, 8) and C % 128 == 0 and C <= 4096
+        # FFN value K parts reduced inside the next layer's LayerNorm
+        parts_ok = splits in LN_PARTS and C % 128 == 0 and C <= 4096
         for l, L in enumerate(m.layers):
             first = l == 0
             P = s.pw[l]
