@@ -1,5 +1,6 @@
 """The decode GEMM's choice of tile by the workgroups it makes (32 x 32 to 128 x 64, eight and four
 waves, whole K and K parts) against the float64 oracle, on each side of its lines."""
+import numpy as np
 import pytest
 import torch
 
@@ -51,3 +52,31 @@ def test_parts(gpu, M, N, K, splits):
     ref, abs_sum = R.gemm(a, w, "nk")
     check(c, ref, ACC * abs_sum, f"{M}x{N}x{K}/{splits}")
     assert (buf[floats:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,C,ranks", [
+    (8, 768, (64, 64, 128)),       # 32 x 32: all of it in one round
+    (65, 1024, (64, 64, 128)),     # short K, more than one round: 32 x 64 with four waves, a step each
+    (129, 2048, (96, 96, 256)),
+    (256, 4096, (128, 128, 480)),  # K of four steps
+])
+def test_low_rank_outputs_batch(gpu, M, C, ranks):
+    """The decode step's low-rank outputs in one launch (bias, none, none, value residual), K up to 512."""
+    ks = [*ranks, 64]
+    a, w = [h(M, k) for k in ks], [h(C, k, scale=0.1) for k in ks]
+    v, vf, v0, w0 = h(M, C), h(M, C), h(C), h(C)
+    tv, tvf, tv0, tw0 = (torch.from_numpy(x).to(gpu) for x in (v, vf, v0, w0))
+    pa, pw = [pack(x, gpu, M, k) for x, k in zip(a, ks)], [pack(x, gpu, C, k) for x, k in zip(w, ks)]
+    c = [torch.full((M, C), float("nan"), dtype=torch.float16, device=gpu) for _ in ks]
+    fp = capi.frag_problem
+    capi.frag_gemm([fp(pa[0], pw[0], c[0], M, C, ks[0], epilogue=capi.EPI_BIAS, v0=tw0),
+                    fp(pa[1], pw[1], c[1], M, C, ks[1]), fp(pa[2], pw[2], c[2], M, C, ks[2]),
+                    fp(pa[3], pw[3], c[3], M, C, ks[3], epilogue=capi.EPI_VALUE_RESIDUAL, v=tv, v_first=tvf, v0=tv0)])
+    z, abs_sum = R._f(a[0]) @ R._f(w[0]).T, np.abs(R._f(a[0])) @ np.abs(R._f(w[0])).T
+    check(c[0], (z + R._f(w0)).astype(np.float16), ACC * abs_sum, "bias")
+    for i in (1, 2):
+        ref, abs_sum = R.gemm(a[i], w[i], "nk")
+        check(c[i], ref, ACC * abs_sum, f"problem {i}")
+    ref, abs_sum = R.gemm(a[3], w[3], "nk", epi="vres", v=v, v_first=vf, v0=v0)
+    # the gate's slope (1/4 of |v_first - v|) times the accumulation error, and the gate's own fp32 rounding
+    check(c[3], ref, 0.25 * np.abs(R._f(vf) - R._f(v)) * ACC * abs_sum + 2e-6, "value residual")
