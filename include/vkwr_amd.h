@@ -366,6 +366,25 @@ VKWR_EXPORT int64_t vkwr_gemm_f16_workspace_bytes(int n_problems, const vkwr_gem
  * that serve every batch size up to a limit.  -1 on invalid arguments. */
 VKWR_EXPORT int64_t vkwr_gemm_f16_workspace_bytes_upto(int n_problems, const vkwr_gemm_problem* problems);
 
+/* Which kernel vkwr_gemm_f16 runs a batch on with a workspace of that many bytes (planning only: it
+ * reads sizes and pointer alignments).  path: one of VKWR_GEMM_PATH_*; tile_m, tile_n: rows and
+ * columns of an output tile (GEMV: tile_m activation rows); parts: most K parts of an output (0: the
+ * large-M path's balanced pieces); scratch_bytes: what it writes of the workspace.  For tests, which
+ * would otherwise not know what they run, and for reading profiles. */
+enum {
+  VKWR_GEMM_PATH_TILE = 0,  /* operands off 16 bytes, K or N off 8 */
+  VKWR_GEMM_PATH_GEMV = 1,  /* up to 4 rows */
+  VKWR_GEMM_PATH_SMALL = 2, /* up to 128 rows */
+  VKWR_GEMM_PATH_MID = 3,
+  VKWR_GEMM_PATH_LARGE = 4
+};
+typedef struct vkwr_gemm_route {
+  int path, tile_m, tile_n, parts;
+  int64_t scratch_bytes;
+} vkwr_gemm_route;
+VKWR_EXPORT int vkwr_gemm_f16_route(int n_problems, const vkwr_gemm_problem* problems, int64_t workspace_bytes,
+                                    vkwr_gemm_route* route);
+
 /* Runs 1..8 independent GEMMs in one launch on the gfx950 matrix cores.
  * `problems` is a host array; `workspace` is device memory of at least
  * vkwr_gemm_f16_workspace_bytes(...) bytes (may be NULL when that is 0).

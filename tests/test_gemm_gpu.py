@@ -296,57 +296,78 @@ def test_cmix_down_relu_one_sparse_shapes(gpu):
 
 # ---------------------------------------------------------------- large-M path
 
-def _big_vs_rowmajor(gpu, shapes, epis, seed):
-    """One launch over `shapes` ([N,K] weights: the 256x256 large-M kernel when eligible) and
-    the same launch over the transposed [K,N] copies (never eligible: the row-major kernel,
-    unsplit for M > 256).  Both feed the same MFMA operands in the same k order from zero
-    and apply the same epilogue arithmetic, so the results are the same bits."""
+def _off(x):
+    """x on memory off 16-byte alignment: a launch with such an operand takes the row-major tile kernel."""
+    y = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:].view(x.shape)
+    return y.copy_(x)
+
+
+def _vs_rowmajor(gpu, shapes, epis, seed, path):
+    """One launch over `shapes` ([N,K] weights), which must take the path named, and the same
+    launch with A off 16-byte alignment, which takes the row-major tile kernel, unsplit.  Both feed the
+    same MFMA operands in the same k order from zero and apply the same epilogue arithmetic, so
+    where the first does not split K either the results are the same bits."""
     from vkwr_amd import capi
     outs = []
-    for layout in (capi.GEMM_B_NK, capi.GEMM_B_KN):
+    for off in (False, True):
         probs, keep = [], []
         for i, ((M, K, N), epi) in enumerate(zip(shapes, epis)):
-            g = torch.Generator(device=gpu).manual_seed(seed + 1000 * i)  # same tensors for both layouts
+            g = torch.Generator(device=gpu).manual_seed(seed + 1000 * i)  # same tensors for both launches
             a = torch.randn(M, K, device=gpu, generator=g).half()
             w = (torch.randn(N, K, device=gpu, generator=g) * 0.05).half()
             c = torch.empty(M, N, dtype=torch.float16, device=gpu)
             v = torch.randn(M, N, device=gpu, generator=g).half()
             vf = torch.randn(M, N, device=gpu, generator=g).half()
             v0 = torch.randn(N, device=gpu, generator=g).half()
-            b = w if layout == capi.GEMM_B_NK else w.t().contiguous()
-            probs.append(capi.gemm_problem(a, b, c, b_layout=layout, epilogue=epi, v=v, v_first=vf, v0=v0))
-            keep += [a, b, c, v, vf, v0]
+            a = _off(a) if off else a
+            probs.append(capi.gemm_problem(a, w, c, epilogue=epi, v=v, v_first=vf, v0=v0))
+            keep += [a, w, c, v, vf, v0]
         ws = torch.empty(max(capi.gemm_workspace_bytes(probs), 0), dtype=torch.uint8, device=gpu)
+        route = capi.gemm_route(probs)
+        assert (route.path, route.parts) == ("tile", 1) if off else route.path == path, route
         capi.gemm(probs, ws)
         torch.cuda.synchronize()
         outs.append([keep[i * 6 + 2].clone() for i in range(len(shapes))])
     return outs
 
 
-@pytest.mark.parametrize("shapes,epis", [
-    ([(300, 1024, 768)], [0]),
-    ([(257, 64, 1000)], [1]),                        # one row past a tile, K of one stage, relu^2
-    ([(768, 448, 1280)], [3]),                       # 15 tiles (not a multiple of the 8 XCDs), bias
-    ([(600, 512, 700), (600, 512, 96), (600, 512, 256), (600, 512, 512)], [1, 0, 3, 2]),  # mixed epilogues
-    ([(2304, 4096, 4096)], [0]),                     # the 7B o-projection shape: 192-row tiles (192 of them)
-    ([(2304, 128, 4096), (2304, 512, 4096)], [3, 2]),  # 7B low-rank outputs: bias, value residual
+@pytest.mark.parametrize("shapes,epis,path", [
+    ([(300, 1024, 768)], [0], "mid"),
+    ([(257, 64, 1000)], [1], "mid"),                 # one row past a tile, K of one stage, relu^2
+    ([(768, 448, 1280)], [3], "mid"),                # bias
+    # N = 700 is no multiple of 8: the row-major kernel, with 16-byte and with single loads
+    ([(600, 512, 700), (600, 512, 96), (600, 512, 256), (600, 512, 512)], [1, 0, 3, 2], "tile"),
+    ([(2304, 4096, 4096)], [0], "large"),            # the 7B o-projection shape: 192-row tiles (192 of them)
+    ([(2304, 128, 4096), (2304, 512, 4096)], [3, 2], "large"),  # 7B low-rank outputs: bias, value residual
+    ([(777, 64, 10248)], [1], "large"),              # K of one stage, ragged in both, 205 tiles of 192 rows
+    ([(2305, 64, 5128)], [3], "large"),              # one row past a tile, 210 tiles of 256 rows
+    ([(1300, 448, 6152)], [0], "large"),             # ragged in both, 175 tiles
+    ([(1025, 64, 6152), (1025, 64, 96), (1025, 64, 256), (1025, 64, 520)], [1, 0, 3, 2], "large"),  # mixed epilogues
+    ([(1537, 256, 4104), (1537, 256, 520)], [4, 5], "large"),  # tanh, sigmoid
+    ([(1300, 64, 3080), (1300, 192, 3080)], [3, 2], "large"),  # unequal K, 91 tiles each (not dealt out by XCD)
+    ([(333, 480, 1000)], [2], "mid"),                # a ragged last stage
+    ([(640, 72, 32776)], [3], "mid"),                # 128 x 256 tiles
 ])
-def test_big_gemm_bitwise_equals_rowmajor_kernel(gpu, shapes, epis):
-    """Launches whose tiles all run whole (no k-parts), in 256- or 192-row tiles: the same bits as
-    the row-major kernel."""
-    big, ref = _big_vs_rowmajor(gpu, shapes, epis, seed=11)
+def test_big_gemm_bitwise_equals_rowmajor_kernel(gpu, shapes, epis, path):
+    """Launches whose tiles all run whole (no k-parts), in the large-M kernel's 256- or 192-row tiles or the
+    mid-size kernel's: the same bits as the row-major kernel."""
+    big, ref = _vs_rowmajor(gpu, shapes, epis, 11, path)
     for i, (x, y) in enumerate(zip(big, ref)):
         assert torch.equal(x, y), (shapes[i], epis[i], float((x.float() - y.float()).abs().max()))
 
 
-def test_big_gemm_split_small_batch_tanh_sigmoid(gpu):
-    """The 7B low-rank inputs alone (w1 padded to 128 columns with tanh, g1 to 512 with sigmoid):
-    36 tiles of 192 rows, each split into k-parts (fp32 partials, ordered fixup): within one fp16
-    ulp plus the fp32 re-association bound of the row-major kernel's result (the activations'
-    slopes are at most 1), and run-to-run identical."""
-    shapes, epis = [(2304, 4096, 128), (2304, 4096, 512)], [4, 5]
-    big, ref = _big_vs_rowmajor(gpu, shapes, epis, seed=11)
-    big2, _ = _big_vs_rowmajor(gpu, shapes, epis, seed=11)
+@pytest.mark.parametrize("shapes,path", [
+    # the 7B low-rank inputs alone (w1 padded to 128 columns with tanh, g1 to 512 with sigmoid)
+    ([(2304, 4096, 128), (2304, 4096, 512)], "mid"),
+    # a whole round of 256-row tiles and 17 more in four k-parts (fp32 partials, ordered fixup)
+    ([(3073, 2048, 1000), (3073, 2048, 4104)], "large"),
+])
+def test_big_gemm_split_small_batch_tanh_sigmoid(gpu, shapes, path):
+    """Tanh and sigmoid epilogues: within one fp16 ulp plus the fp32 re-association bound of the row-major
+    kernel's result (the activations' slopes are at most 1), and run-to-run identical."""
+    epis = [4, 5]
+    big, ref = _vs_rowmajor(gpu, shapes, epis, 11, path)
+    big2, _ = _vs_rowmajor(gpu, shapes, epis, 11, path)
     for i, (M, K, N) in enumerate(shapes):
         g = torch.Generator(device=gpu).manual_seed(11 + 1000 * i)
         a = torch.randn(M, K, device=gpu, generator=g).half()
@@ -360,8 +381,8 @@ def test_big_gemm_split_small_batch_tanh_sigmoid(gpu):
         assert torch.equal(big[i], big2[i])
 
 
-@pytest.mark.parametrize("M,K,N", [(300, 256, 200), (2304, 512, 256)])
-def test_tanh_sigmoid_epilogues(gpu, M, K, N):
+@pytest.mark.parametrize("M,K,N,path", [(300, 256, 200, "mid"), (2304, 512, 256, "mid"), (777, 64, 10248, "large")])
+def test_tanh_sigmoid_epilogues(gpu, M, K, N, path):
     """c = tanh(a b^T) and sigmoid(a b^T), fp32 accumulation, against torch in float64."""
     from vkwr_amd import capi
     g = torch.Generator(device=gpu).manual_seed(M + N)
@@ -371,6 +392,7 @@ def test_tanh_sigmoid_epilogues(gpu, M, K, N):
     for epi, fn in ((capi.EPI_TANH, torch.tanh), (capi.EPI_SIGMOID, torch.sigmoid)):
         c = torch.empty(M, N, dtype=torch.float16, device=gpu)
         p = [capi.gemm_problem(a, w, c, epilogue=epi)]
+        assert capi.gemm_route(p).path == path
         ws = torch.empty(max(capi.gemm_workspace_bytes(p), 0), dtype=torch.uint8, device=gpu)
         capi.gemm(p, ws)
         torch.cuda.synchronize()
@@ -378,17 +400,21 @@ def test_tanh_sigmoid_epilogues(gpu, M, K, N):
         assert (c.double() - fn(ref)).abs().max().item() <= 2e-3
 
 
-def test_big_gemm_batch_with_empty_problem_and_oracle(gpu):
+@pytest.mark.parametrize("shapes,path", [
+    ([(384, 256, 520), (0, 256, 64), (384, 256, 200)], "mid"),
+    ([(1300, 256, 5128), (0, 256, 64), (1300, 256, 520)], "large"),
+])
+def test_big_gemm_batch_with_empty_problem_and_oracle(gpu, shapes, path):
     """A launch whose batch holds an empty problem between eligible ones; every output against
     the float64 oracle."""
     from vkwr_amd import capi
-    shapes = [(384, 256, 520), (0, 256, 64), (384, 256, 200)]
     a = [h(M, K) for M, K, N in shapes]
     w = [h(N, K, scale=0.05) for M, K, N in shapes]
     da = [dev(x, gpu) for x in a]
     dw = [dev(x, gpu) for x in w]
     c = [torch.full((M, N), float("nan"), dtype=torch.float16, device=gpu) for M, K, N in shapes]
     probs = [capi.gemm_problem(x, y, z) for x, y, z in zip(da, dw, c)]
+    assert capi.gemm_route(probs).path == path
     capi.gemm(probs, torch.empty(0, dtype=torch.uint8, device=gpu))
     torch.cuda.synchronize()
     for i, (M, K, N) in enumerate(shapes):
@@ -425,44 +451,47 @@ def test_small_m_kn_fragments_equal_nk_bitwise(gpu, M, K, N):
     assert torch.equal(out[0], out[1])
 
 
-@pytest.mark.parametrize("M,K,N", [
-    (1024, 16384, 2048),   # 32 tiles, long K: every tile split into 8 k-parts
-    (2304, 16384, 4096),   # the 7B FFN value shape: 144 tiles of 256 stages, layered split
-                           # (144 stages per CU: [0, 144) of every tile, [144, 256) of 112 tiles
-                           # whole, the other 32 in 16-stage pieces)
-    (2304, 8192, 4096),    # 144 tiles of 128 stages: per 72, layered with 8-stage pieces
-    (4096, 16384, 6400),   # 400 tiles: 256 whole, the other 144 layered (tile indices offset by 256)
-    (2304, 4096, 8192),    # 288 tiles: one whole round + a 32-tile tail split in 6
-    (2304, 4096, 16384),   # the 7B FFN key shape: 768 whole 192-row tiles (three rounds, no split)
+@pytest.mark.parametrize("M,K,N,path,parts", [
+    (1024, 16384, 2048, "mid", 4),     # 256 x 128 tiles, long K in four parts
+    (2304, 16384, 4096, "large", 0),   # the 7B FFN value shape: 144 tiles of 256 stages, layered split
+                                       # (144 stages per CU: [0, 144) of every tile, [144, 256) of 112 tiles
+                                       # whole, the other 32 in 16-stage pieces)
+    (2304, 8192, 4096, "large", 1),    # 192 whole tiles of 192 rows
+    (4096, 16384, 6400, "large", 0),   # 400 tiles: 256 whole, the other 144 layered (tile indices offset by 256)
+    (2304, 4096, 8192, "large", 6),    # 288 tiles: one whole round + a 32-tile tail split in 6
+    (2304, 4096, 16384, "large", 1),   # the 7B FFN key shape: 768 whole 192-row tiles (three rounds, no split)
+    (1537, 2048, 10248, "large", 4),   # 287 tiles, ragged in both: a 31-tile tail in 4
+    (1000, 2048, 16392, "large", 4),   # 260 tiles: a tail of 4
 ])
-def test_big_gemm_split_tail(gpu, M, K, N):
+def test_big_gemm_split_tail(gpu, M, K, N, path, parts):
     """Tail tiles split into k-parts or balanced pieces (fp32 partials, ordered fixup): against the row-major
-    kernel on the transposed weight within the fp32 re-association bound, and run-to-run
+    kernel (A off 16-byte alignment) within the fp32 re-association bound, and run-to-run
     bitwise identical (also through the relu^2 epilogue)."""
     from vkwr_amd import capi
     g = torch.Generator(device=gpu).manual_seed(M + K + N)
     a = torch.randn(M, K, device=gpu, generator=g).half()
     w = (torch.randn(N, K, device=gpu, generator=g) * 0.02).half()
-    wt = w.t().contiguous()
 
-    def run(b, layout, epi=capi.EPI_NONE):
+    def run(a, epi=capi.EPI_NONE, want=(path, parts)):
         c = torch.empty(M, N, dtype=torch.float16, device=gpu)
-        p = [capi.gemm_problem(a, b, c, b_layout=layout, epilogue=epi)]
+        p = [capi.gemm_problem(a, w, c, epilogue=epi)]
+        route = capi.gemm_route(p)
+        assert (route.path, route.parts) == want, route
         ws = torch.empty(max(capi.gemm_workspace_bytes(p), 0), dtype=torch.uint8, device=gpu)
         capi.gemm(p, ws)
         return c
 
-    nk = run(w, capi.GEMM_B_NK)
-    kn = run(wt, capi.GEMM_B_KN)
+    nk = run(a)
+    rowmajor = run(_off(a), want=("tile", 1))
     abs_sum = (a.abs().float() @ w.abs().float().t())
     torch.cuda.synchronize()
-    ref = kn.double()
+    ref = rowmajor.double()
     ulp = torch.exp2(torch.floor(torch.log2(ref.abs().clamp_min(2.0 ** -14))) - 10)
     bound = ulp + ACC * abs_sum.double()
     err = (nk.double() - ref).abs()
     assert bool((err <= bound).all()), (float(err.max()), int((err > bound).sum()))
-    r1 = run(w, capi.GEMM_B_NK, capi.EPI_RELU_SQUARE)
-    r2 = run(w, capi.GEMM_B_NK, capi.EPI_RELU_SQUARE)
+    r1 = run(a, capi.EPI_RELU_SQUARE)
+    r2 = run(a, capi.EPI_RELU_SQUARE)
     torch.cuda.synchronize()
     assert torch.equal(r1, r2)
 

@@ -44,19 +44,25 @@ def _run_ws(probs, gpu):
 
 
 @pytest.mark.parametrize("shapes", [
-    # (m, n, k, epilogue, problems, [K,N] weights): a K-split batch, then a smaller one
-    [(128, 1024, 8192, capi.EPI_NONE, 1, False), (40, 1024, 2048, capi.EPI_BIAS, 3, False)],
-    # the large-M kernel's split last round (stream-K partials), then a smaller split batch
-    [(500, 4096, 2048, capi.EPI_RELU_SQUARE, 1, False), (64, 1024, 4096, capi.EPI_NONE, 2, False)],
+    # (m, n, k, epilogue, problems, [K,N] weights, path): a K-split batch, then a smaller one
+    [(128, 1024, 8192, capi.EPI_NONE, 1, False, "small"), (40, 1024, 2048, capi.EPI_BIAS, 3, False, "small")],
+    # tiles of the mid-size kernel that write no partials (the demand is that of the path they replaced),
+    # then a split batch
+    [(500, 4096, 2048, capi.EPI_RELU_SQUARE, 1, False, "mid whole"), (64, 1024, 4096, capi.EPI_NONE, 2, False, "small")],
+    # the large-M kernel's split last round (stream-K partials), then the mid-size kernel's K parts
+    [(3073, 5128, 2048, capi.EPI_RELU_SQUARE, 1, False, "large"), (700, 264, 8192, capi.EPI_NONE, 2, False, "mid")],
     # the GEMV kernel's K parts ([K,N] weights, M <= 4), then a smaller one
-    [(3, 4096, 4096, capi.EPI_NONE, 1, True), (1, 2048, 2048, capi.EPI_BIAS, 2, True)],
+    [(3, 4096, 4096, capi.EPI_NONE, 1, True, "gemv"), (1, 2048, 2048, capi.EPI_BIAS, 2, True, "gemv")],
 ])
 def test_noalloc_equals_workspace_entry_point(gpu, shapes):
     assert _max() == 32 << 20
-    for i, (m, n, k, epi, npb, kn) in enumerate(shapes):
+    for i, (m, n, k, epi, npb, kn, path) in enumerate(shapes):
         probs, outs, keep = _batch(gpu, m, n, k, seed=10 + i, epilogue=epi, nprob=npb, kn=kn)
         need = capi.gemm_workspace_bytes(probs)
-        assert 0 < need <= _max(), need  # the scratch is really used
+        assert 0 < need <= _max(), need
+        route = capi.gemm_route(probs)
+        # the scratch is really used
+        assert path == "mid whole" and route.path == "mid" or route.path == path and 0 < route.scratch_bytes <= need, route
         _run_noalloc(probs)
         got = [o.clone() for o in outs]
         for o in outs:
@@ -68,12 +74,17 @@ def test_noalloc_equals_workspace_entry_point(gpu, shapes):
             assert torch.equal(g_, w_), (m, n, k)
 
 
-def test_noalloc_rejects_batches_beyond_its_scratch(gpu):
-    """A batch whose plan needs more than the scratch holds fails on the host with a clear
+@pytest.mark.parametrize("m,n,k,path", [
+    (512, 4096, 4096, "mid"),     # runs whole in the mid-size path, which asks for what the path it replaced took
+    (2304, 8192, 4096, "large"),  # 48 MiB of partials
+])
+def test_noalloc_rejects_batches_beyond_its_scratch(gpu, m, n, k, path):
+    """A batch that asks for more than the scratch holds fails on the host with a clear
     message and enqueues nothing."""
-    probs, outs, keep = _batch(gpu, 512, 4096, 4096, seed=3)
+    probs, outs, keep = _batch(gpu, m, n, k, seed=3)
     need = capi.gemm_workspace_bytes(probs)
-    assert need > _max()
+    route = capi.gemm_route(probs)
+    assert need > _max() and route.path == path and (route.scratch_bytes == need if path == "large" else True)
     with pytest.raises(RuntimeError, match="at most"):
         _run_noalloc(probs)
     torch.cuda.synchronize()

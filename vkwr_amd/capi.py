@@ -10,6 +10,7 @@ raises RuntimeError with the library's message.
 """
 import ctypes
 import os
+import types
 
 import torch
 
@@ -49,6 +50,10 @@ class GemmProblem(ctypes.Structure):
                 ("b_layout", _i), ("a_act", _i), ("epilogue", _i), ("v", _p), ("v_first", _p), ("v0", _p)]
 
 
+class GemmRoute(ctypes.Structure):
+    _fields_ = [("path", _i), ("tile_m", _i), ("tile_n", _i), ("parts", _i), ("scratch_bytes", _i64)]
+
+
 class FragProblem(ctypes.Structure):
     _fields_ = [("a", _p), ("b", _p), ("c", _p), ("m", _i64), ("n", _i64), ("k", _i64),
                 ("epilogue", _i), ("c_frag", _i), ("v", _p), ("v_first", _p), ("v0", _p)]
@@ -69,6 +74,7 @@ _LIB.vkwr_last_error.restype = ctypes.c_char_p
 _gemm = _sig("vkwr_gemm_f16", [_i, ctypes.POINTER(GemmProblem), _p, _i64, _p])
 _gemm_ws = _sig("vkwr_gemm_f16_workspace_bytes", [_i, ctypes.POINTER(GemmProblem)], _i64)
 _gemm_ws_upto = _sig("vkwr_gemm_f16_workspace_bytes_upto", [_i, ctypes.POINTER(GemmProblem)], _i64)
+_gemm_route = _sig("vkwr_gemm_f16_route", [_i, ctypes.POINTER(GemmProblem), _i64, ctypes.POINTER(GemmRoute)])
 _ln_mix = _sig("vkwr_add_layer_norm_mix_f16",
                [_i64, _i, _p, _p, _p, _p, _p, _i, ctypes.POINTER(_p), _f, _p, ctypes.POINTER(_p), _p, _p, _i64, _i64,
                 _p])
@@ -165,6 +171,18 @@ def gemm_workspace_bytes(problems):
     if n < 0:
         raise RuntimeError(f"vkwr_gemm_f16_workspace_bytes: {_LIB.vkwr_last_error().decode()}")
     return n
+
+
+def gemm_route(problems, workspace_bytes=None):
+    """The kernel that `gemm` runs this batch on, given its whole workspace or so many bytes of it
+    (vkwr_gemm_f16_route): path ("tile", "gemv", "small", "mid", "large"), tile_m, tile_n, parts,
+    scratch_bytes."""
+    if workspace_bytes is None:
+        workspace_bytes = gemm_workspace_bytes(problems)
+    r = GemmRoute()
+    _check(_gemm_route(len(problems), _arr(problems), workspace_bytes, ctypes.byref(r)), "vkwr_gemm_f16_route")
+    return types.SimpleNamespace(path=("tile", "gemv", "small", "mid", "large")[r.path], tile_m=r.tile_m,
+                                 tile_n=r.tile_n, parts=r.parts, scratch_bytes=r.scratch_bytes)
 
 
 def gemm_workspace_bytes_upto(problems):

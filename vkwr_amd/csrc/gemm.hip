@@ -2512,15 +2512,21 @@ constexpr int kTargetWgs = 512;  // two workgroups per CU on 256 CUs
 
 // Plans the batch with at most `limit` bytes for the mid-size path's K parts.  *need: the
 // workspace to ask for -- the plan's, and never less than the plan of the other paths takes, so
-// that what a workspace (or the fixed scratch) was too small for stays refused.
+// that what a workspace (or the fixed scratch) was too small for stays refused.  *used: what the
+// launch writes of it.
 int plan_batch(const char* fn, int n, const vkwr_gemm_problem* pr, int64_t limit, Batch& bt, Config& cfg, BigPlan& pl,
-               int64_t* need) {
+               int64_t* need, int64_t* used = nullptr) {
   int rows = 0;
   double planned = 0;
   if (int e = build_batch(fn, n, pr, bt, cfg, rows)) return e;
-  *need = cfg.big ? plan_big(bt, pl, &planned) : plan(bt, cfg, kTargetWgs);
+  int64_t own = cfg.big ? plan_big(bt, pl, &planned) : plan(bt, cfg, kTargetWgs);
+  *need = own;
   mid_choose(bt, rows, std::min(limit, kMidMaxWs), pl, planned, cfg);
-  if (cfg.mid) *need = std::max(*need, plan(bt, cfg, kTargetWgs));
+  if (cfg.mid) {
+    own = plan(bt, cfg, kTargetWgs);
+    *need = std::max(*need, own);
+  }
+  if (used) *used = own;
   return VKWR_OK;
 }
 
@@ -2537,6 +2543,26 @@ extern "C" int64_t vkwr_gemm_f16_workspace_bytes(int n_problems, const vkwr_gemm
   int64_t need;
   if (plan_batch("vkwr_gemm_f16_workspace_bytes", n_problems, problems, kMidMaxWs, bt, cfg, pl, &need)) return -1;
   return need;
+}
+
+extern "C" int vkwr_gemm_f16_route(int n_problems, const vkwr_gemm_problem* problems, int64_t workspace_bytes,
+                                   vkwr_gemm_route* route) {
+  clear_error();
+  const char* fn = "vkwr_gemm_f16_route";
+  VK_REQUIRE(route != nullptr, "%s: null route", fn);
+  Batch bt;
+  Config cfg;
+  BigPlan pl;
+  int64_t need, used;
+  if (int e = plan_batch(fn, n_problems, problems, workspace_bytes, bt, cfg, pl, &need, &used)) return e;
+  int parts = 1;
+  if (cfg.big) parts = pl.sk_tiles > 0 ? pl.parts : 1;
+  else
+    for (int i = 0; i < bt.n; ++i) parts = std::max(parts, bt.p[i].splits);
+  *route = vkwr_gemm_route{cfg.mid ? VKWR_GEMM_PATH_MID : cfg.big ? VKWR_GEMM_PATH_LARGE : cfg.gv ? VKWR_GEMM_PATH_GEMV
+                           : cfg.rm ? VKWR_GEMM_PATH_SMALL : VKWR_GEMM_PATH_TILE,
+                           cfg.gv ? cfg.gv : cfg.big ? pl.bm : cfg.bm, cfg.bn, parts, used};
+  return VKWR_OK;
 }
 
 extern "C" int64_t vkwr_gemm_f16_workspace_bytes_upto(int n_problems, const vkwr_gemm_problem* problems) {
