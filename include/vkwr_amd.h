@@ -354,11 +354,14 @@ typedef struct vkwr_gemm_problem {
   const uint16_t* v0;
 } vkwr_gemm_problem;
 
-/* Bytes of device workspace vkwr_gemm_f16 wants for this batch (fp32 partial
- * sums: K splits of small-M and mid-size problems, or the k-parts of a large-M batch's
- * last round of 256x256 tiles; 0 when nothing is split), or -1 on invalid arguments.
- * The plan depends on the current device's CU count: ask on that device.  (Where only the
- * mid-size path would split, vkwr_gemm_f16 with less runs that path in fewer parts.) */
+/* Bytes of device workspace that vkwr_gemm_f16 asks for with this batch, or -1 on invalid arguments:
+ * room for fp32 partial sums (K splits of small-M and mid-size problems, or the k-parts of a
+ * large-M batch's last round of 256x256 tiles; 0 where no path that can take the batch splits it).
+ * A batch that the mid-size path takes over from another still asks for what that one writes, so
+ * that which workspaces are too small does not change with the choice between them;
+ * vkwr_gemm_f16_route tells what the launch writes.  Where only the mid-size path would split,
+ * vkwr_gemm_f16 with less runs that path in fewer parts.
+ * The plan depends on the current device's CU count: ask on that device. */
 VKWR_EXPORT int64_t vkwr_gemm_f16_workspace_bytes(int n_problems, const vkwr_gemm_problem* problems);
 
 /* The largest workspace the batch needs when every problem's m is replaced by the same row
@@ -400,7 +403,7 @@ VKWR_EXPORT int vkwr_gemm_f16(int n_problems, const vkwr_gemm_problem* problems,
  * stream-K partials go to a scratch array of vkwr_gemm_f16_noalloc_max_bytes() bytes
  * (32 MiB) that the library holds in device memory, one copy per device, for the life of
  * the process.  Same plan, same kernels, same results bit for bit as vkwr_gemm_f16 with a
- * workspace.  A batch whose plan needs more scratch (vkwr_gemm_f16_workspace_bytes) than
+ * workspace.  A batch that asks for more (vkwr_gemm_f16_workspace_bytes) than
  * that is rejected with VKWR_ERR_INVALID before any GPU work; every GEMM batch of the
  * 1.5B-shape decode step (C = 2048) at up to 256 rows fits.  It calls no hipMalloc / hipFree.  Calls that overlap on
  * one device (concurrent streams, or host threads) share that device's scratch and race:

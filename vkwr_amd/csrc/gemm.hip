@@ -2397,8 +2397,8 @@ double big_estimate(const Batch& bt, const BigPlan& pl, double planned) {
   return 1.1 * std::max(t, gemm_stream_us(bt));
 }
 
-// Most partials (bytes) a mid-size plan may take: the scratch of vkwr_gemm_f16_noalloc.
-constexpr int64_t kMidMaxWs = (int64_t)32 << 20;
+// Scratch that vkwr_gemm_f16_noalloc holds, and so the most partials (bytes) a mid-size plan may take.
+constexpr int64_t kNoAllocScratchBytes = (int64_t)32 << 20;
 
 // Moves the batch to gemm_mid_kernel where that is faster than `cfg`, the path chosen among
 // the others; `limit` bounds the workspace of its K parts.
@@ -2511,9 +2511,10 @@ int build_batch(const char* fn, int n, const vkwr_gemm_problem* pr, Batch& bt, C
 constexpr int kTargetWgs = 512;  // two workgroups per CU on 256 CUs
 
 // Plans the batch with at most `limit` bytes for the mid-size path's K parts.  *need: the
-// workspace to ask for -- the plan's, and never less than the plan of the other paths takes, so
-// that what a workspace (or the fixed scratch) was too small for stays refused.  *used: what the
-// launch writes of it.
+// workspace to ask for -- the plan's, and where the mid-size path took the batch over no less than
+// the path it replaced takes (512 x 4096 x 4096: 45 MiB of which nothing is written), so that a call that
+// a workspace or the fixed scratch is too small for does not depend on the time models.  *used: what
+// the launch writes of it.
 int plan_batch(const char* fn, int n, const vkwr_gemm_problem* pr, int64_t limit, Batch& bt, Config& cfg, BigPlan& pl,
                int64_t* need, int64_t* used = nullptr) {
   int rows = 0;
@@ -2521,7 +2522,7 @@ int plan_batch(const char* fn, int n, const vkwr_gemm_problem* pr, int64_t limit
   if (int e = build_batch(fn, n, pr, bt, cfg, rows)) return e;
   int64_t own = cfg.big ? plan_big(bt, pl, &planned) : plan(bt, cfg, kTargetWgs);
   *need = own;
-  mid_choose(bt, rows, std::min(limit, kMidMaxWs), pl, planned, cfg);
+  mid_choose(bt, rows, std::min(limit, kNoAllocScratchBytes), pl, planned, cfg);
   if (cfg.mid) {
     own = plan(bt, cfg, kTargetWgs);
     *need = std::max(*need, own);
@@ -2541,7 +2542,7 @@ extern "C" int64_t vkwr_gemm_f16_workspace_bytes(int n_problems, const vkwr_gemm
   Config cfg;
   BigPlan pl;
   int64_t need;
-  if (plan_batch("vkwr_gemm_f16_workspace_bytes", n_problems, problems, kMidMaxWs, bt, cfg, pl, &need)) return -1;
+  if (plan_batch("vkwr_gemm_f16_workspace_bytes", n_problems, problems, kNoAllocScratchBytes, bt, cfg, pl, &need)) return -1;
   return need;
 }
 
@@ -2572,12 +2573,12 @@ extern "C" int64_t vkwr_gemm_f16_workspace_bytes_upto(int n_problems, const vkwr
   Config cfg;
   BigPlan pl;
   int64_t need, most = 0;
-  if (plan_batch(fn, n_problems, problems, kMidMaxWs, bt, cfg, pl, &need)) return -1;
+  if (plan_batch(fn, n_problems, problems, kNoAllocScratchBytes, bt, cfg, pl, &need)) return -1;
   vkwr_gemm_problem p[kMaxProblems];
   std::copy(problems, problems + n_problems, p);
   for (int64_t m = 1; m <= problems[0].m; ++m) {
     for (int i = 0; i < n_problems; ++i) p[i].m = m;
-    if (plan_batch(fn, n_problems, p, kMidMaxWs, bt, cfg, pl, &need)) return -1;
+    if (plan_batch(fn, n_problems, p, kNoAllocScratchBytes, bt, cfg, pl, &need)) return -1;
     most = std::max(most, need);
   }
   return most;
@@ -2587,7 +2588,6 @@ extern "C" int64_t vkwr_gemm_f16_workspace_bytes_upto(int n_problems, const vkwr
 // device that loads the library holds its own copy for the life of the process.  Host code
 // reaches it only through the address hipGetSymbolAddress returns for the current device
 // (scratch_ptr below); the array's name itself is a host-side stand-in.
-static constexpr int64_t kNoAllocScratchBytes = (int64_t)32 << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
