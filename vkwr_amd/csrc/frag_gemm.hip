@@ -382,7 +382,7 @@ int tiles_for(const FBatch& bt, int bm, int bn) {
 
 // One configuration per launch; `splits` K parts per tile.
 //
-// The smallest tile whose workgroups fit the 256 CUs at once: a second round of workgroups costs more
+// The smallest tile whose workgroups fit the (256) CUs at once: a second round of workgroups costs more
 // than larger tiles that leave some CUs idle, and half as many workgroups as CUs leave bandwidth.
 // us, this tile against the others (proj: three [C, C] and four low-rank problems in a launch):
 //   32 x 32    K 2048, N 8192, m <= 32    8.9; 32 x 64 11.0, 64 x 64 12.8
@@ -418,10 +418,11 @@ FragConfig pick_frag_config(const FBatch& bt, int splits) {
     while (ks > 1 && kdiv % (16 * ks * nw) != 0) ks /= 2;
     return ks;
   };
-  auto fits = [&](int bm, int bn) { return (int64_t)tiles_for(bt, bm, bn) * splits <= 256; };
+  const int cus = device_cus();
+  auto fits = [&](int bm, int bn) { return (int64_t)tiles_for(bt, bm, bn) * splits <= cus; };
   if (fits(32, 32)) return {1, 1, 8, ks_for(8, 4)};
   if (splits == 1 && max_k <= 512) return {1, 2, 4, 1};
-  if (splits == 1 && max_k <= 1024 && tiles_for(bt, 32, 32) <= 768) return {1, 1, 8, ks_for(8, 4)};
+  if (splits == 1 && max_k <= 1024 && tiles_for(bt, 32, 32) <= 3 * cus) return {1, 1, 8, ks_for(8, 4)};
   if (fits(32, 64)) return {1, 2, 8, ks_for(8, 2)};
   if (fits(64, 64)) return {2, 2, 8, ks_for(8, 2)};
   if (fits(128, 64)) return {4, 2, 4, ks_for(4, 2)};
