@@ -433,8 +433,8 @@ def wkv_fp16_family(dev, steps, seq_calls=20, warmup=5):
         "kernel": "wkv7_fp16_quad_kernel<false>: T >= 4 with at most one chain per CU"}
     del r, w, k, v, a, b, st, yp
     torch.cuda.empty_cache()
-    out["kernel"] = ("wkv7_fp16_kernel<false> (T = 1) and wkv7_fp16_quad_kernel<false> (T > 1, few chains), "
-                     "vkwr_amd/csrc/wkv.hip: one wave64 (T = 1) or four (T > 1) per (sequence, head)")
+    out["kernel"] = ("wkv7_fp16_kernel<false> (T = 1) and wkv7_fp16_quad_kernel<false> (T >= 4, at most one chain per CU), "
+                     "vkwr_amd/csrc/wkv.hip: one wave64 or four per (sequence, head)")
     out["timing"] = "decode: HIP graph of the steps, HIP events on the replay stream; prefill: eager calls"
     return out
 

@@ -2000,7 +2000,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   }
 }
 
-// The same recurrence for T > 1 with one workgroup per CU or fewer: four waves per (sequence,
+// The same recurrence for T >= 4 with at most one chain per CU and 16-byte aligned rows: four waves per (sequence,
 // head), so that a lone wave's 160 FMAs per token become ~90 on each of the four SIMDs.
 //
 // Wave w owns rows 16 w .. 16 w + 15; the four lanes of a quad hold one row, lane cg of it columns 16
