@@ -771,7 +771,7 @@ __global__ __launch_bounds__(256) void wkv7_fp32_rows_kernel(RowsArgs ra) {
 // Pipeline (one barrier per chunk): in iteration c the state waves run chunk c against the
 // state (Â X0^T, R̂ X0^T, K̂^T V, then Z = W RHS, Y and B̂^T Z: the dependent chain of a
 // chunk), while matrix waves 4-7 prepare chunk c + 3's hat vectors (VALU work: Λ by a
-// DPP scan of the log decays over the 16 lanes that hold one channel quad's tokens), chunk
+// DPP scan of the decays over the 16 lanes that hold one channel quad's tokens), chunk
 // c + 2's four L x L matrices and chunk c + 1's W^T from its N (described at the kernel).
 // Per chunk: 80 MFMAs on each state wave, 116 / 112 / 96 / 96 on the four SIMDs.  Measured
 // at config 2: 0.174 ms per call (0.24 ms for the form with four waves, each running all
@@ -808,8 +808,11 @@ __device__ __forceinline__ float log2_decay_fast(float w) {
 typedef const __attribute__((address_space(1))) hv8 global_hv8;
 
 // x + (the value of the lane `n` below in the same 16-lane row, 0 for the first n lanes)
+// (multiplied: 1 for them)
 #define VK_SCAN_ADD(x, ctrl) \
   x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), ctrl, 0xF, 0xF, false))
+#define VK_SCAN_MUL(x, ctrl) \
+  x *= __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, 1.0f), __builtin_bit_cast(int, x), ctrl, 0xF, 0xF, false))
 
 struct ChunkLds {
   // fp16 r, w, k, v, a, b: [vec][t][8 x 8 channels + 8 of padding].  The padding spreads the
@@ -838,8 +841,8 @@ struct ChunkLds {
 //      matrices) and the final state;
 //   3. wkv_seg_out_kernel: y = y0 + S_start q, all tokens at once.
 // Everything between the launches is fp32.  The products of step 2 and 3 only re-associate the
-// sums of the one-chain form: against 64 bits the state is off by 3.4e-7 (one chain 2.7e-7; 3.8e-7
-// with Λ formed as a product), y by its fp16 rounding.  T is taken in blocks of `len` tokens so
+// sums of the one-chain form: against 64 bits the state is off by 3.4e-7 after 1500 tokens of decays from
+// 0.6 to 0.998 (one chain 2.8e-7), y by its fp16 rounding.  T is taken in blocks of `len` tokens so
 // that the scratch stays bounded.  What bounds it: 3.4 us per chunk of a segment (the state waves'
 // products) and ~26 us of pipeline fill and launches; 32 chains, T = 1500: 217 -> 77 us.
 //
@@ -975,16 +978,20 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra, SegAr
     float l1[4], l0[4], rl[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      // Λ_t = 2^(sum of the log decays): one rounding of an exp2 per token of the chunk instead of
-      // the product's one per factor (state off 64 bits by 2.7e-7 instead of 3.8e-7 over 1500 tokens), at the
-      // same number of instructions
+      // Λ_t: the log decays summed over windows of four tokens, then the windows' exp2 multiplied.  Long
+      // memory wants sums (a decay near 1 loses its distance from it in fp32), short memory products (a
+      // sum of 16 goes to 14 and rounds by 5e-7, all of it relative error of Λ).  State against 64 bits, 48
+      // tokens, products / this / sums throughout: w = 2 + N 1.47e-7, 1.72e-7, 2.77e-7; tanh N 1.62e-7, 1.65e-7, 2.06e-7;
+      // -6 .. -1 by channel 3.55e-7, 2.86e-7, 2.74e-7; -8 9.2e-7, 5.9e-7, 2.8e-7.  Exact sums (the
+      // logs split in two) have the least of all, 1.27e-7 to 2.8e-7, and cost 6 % of a prefill.
       float d = in * log2_decay_fast((float)x.w[e]);
       VK_SCAN_ADD(d, 0x111);  // row_shr:1
       VK_SCAN_ADD(d, 0x112);  // row_shr:2
-      VK_SCAN_ADD(d, 0x114);  // row_shr:4
-      VK_SCAN_ADD(d, 0x118);  // row_shr:8
-      l1[e] = __builtin_amdgcn_exp2f(d);   // Λ_t
-      rl[e] = __builtin_amdgcn_exp2f(-d);  // 1 / Λ_t
+      d = __builtin_amdgcn_exp2f(d);
+      VK_SCAN_MUL(d, 0x114);  // row_shr:4
+      VK_SCAN_MUL(d, 0x118);  // row_shr:8
+      l1[e] = d;
+      rl[e] = __builtin_amdgcn_rcpf(d);
       l0[e] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, 1.0f),
                                                                      __builtin_bit_cast(int, l1[e]), 0x111, 0xF, 0xF, false));
     }
