@@ -807,8 +807,7 @@ __device__ __forceinline__ float log2_decay_fast(float w) {
 
 typedef const __attribute__((address_space(1))) hv8 global_hv8;
 
-// x + (the value of the lane `n` below in the same 16-lane row, 0 for the first n lanes)
-// (multiplied: 1 for them)
+// x + (x *) the value of the lane `n` below in the same 16-lane row, 0 (1) for the first n lanes
 #define VK_SCAN_ADD(x, ctrl) \
   x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), ctrl, 0xF, 0xF, false))
 #define VK_SCAN_MUL(x, ctrl) \
