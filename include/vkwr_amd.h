@@ -546,6 +546,15 @@ typedef struct vkwr_frag_gemm_problem {
 VKWR_EXPORT int vkwr_frag_gemm_f16(int n_problems, const vkwr_frag_gemm_problem* problems,
                                    void* stream);
 
+/* The tile (rows, columns), waves per workgroup and workgroups that vkwr_frag_gemm_f16 runs a batch with, or
+ * with splits > 1 vkwr_frag_gemm_splitk_f16 its one problem (planning only).  For tests and for reading
+ * profiles. */
+typedef struct vkwr_frag_gemm_route {
+  int tile_m, tile_n, waves, workgroups;
+} vkwr_frag_gemm_route;
+VKWR_EXPORT int vkwr_frag_gemm_f16_route(int n_problems, const vkwr_frag_gemm_problem* problems, int splits,
+                                         vkwr_frag_gemm_route* route);
+
 /* One frag GEMM with K split over `splits` workgroups per output
  * tile: the parts write fp32 partial tiles to `workspace`, and a second
  * kernel adds them in increasing K order and applies the epilogue (same

@@ -59,6 +59,10 @@ class FragProblem(ctypes.Structure):
                 ("epilogue", _i), ("c_frag", _i), ("v", _p), ("v_first", _p), ("v0", _p)]
 
 
+class FragRoute(ctypes.Structure):
+    _fields_ = [("tile_m", _i), ("tile_n", _i), ("waves", _i), ("workgroups", _i)]
+
+
 class LnShiftGroup(ctypes.Structure):
     _fields_ = [("row0", _i64), ("B", ctypes.c_int32), ("T", ctypes.c_int32), ("slots", _p)]
 
@@ -90,6 +94,7 @@ _wkv_prefill_ws = _sig("vkwr_wkv7_fp32_prefill_workspace_bytes", [_i, _i, _i], _
 _wkv_prefill_max = _sig("vkwr_wkv7_fp32_prefill_workspace_max", [_i64, _i], _i64)
 _wkv_step_rows = _sig("vkwr_wkv7_fp32_step_rows_slots", [_i, _i, _i, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p])
 _frag_gemm = _sig("vkwr_frag_gemm_f16", [_i, ctypes.POINTER(FragProblem), _p])
+_frag_route = _sig("vkwr_frag_gemm_f16_route", [_i, ctypes.POINTER(FragProblem), _i, ctypes.POINTER(FragRoute)])
 _act = _sig("vkwr_activation_f16", [_i, _i64, _p, _p, _p])
 ACT_EW_TANH, ACT_EW_SIGMOID = 1, 2  # vkwr_activation_f16 codes
 _frag_splitk = _sig("vkwr_frag_gemm_splitk_f16", [ctypes.POINTER(FragProblem), _i, _p, _i64, _p])
@@ -316,6 +321,14 @@ def add_layer_norm_mix_parts(x_parts, n_parts, part_stride, residual, shift_stat
                          _ptr(weight), _ptr(bias), len(mixes), mp, eps, _ptr(x_out), op,
                          _idx(shift_slots, rows, "shift_slots"),
                          shift_state.numel() // C, _stream()), "vkwr_add_layer_norm_mix_parts_frag_f16")
+
+
+def frag_route(problems, splits=1):
+    """The tile that `frag_gemm` (splits = 1) or the K-split form runs with (vkwr_frag_gemm_f16_route):
+    (tile_m, tile_n, waves, workgroups)."""
+    r = FragRoute()
+    _check(_frag_route(len(problems), _arr_frag(problems), splits, ctypes.byref(r)), "vkwr_frag_gemm_f16_route")
+    return r.tile_m, r.tile_n, r.waves, r.workgroups
 
 
 def _arr_frag(problems):

@@ -392,16 +392,23 @@ int tiles_for(const FBatch& bt, int bm, int bn) {
 //   128 x 64   the same, m = 160 - 256   17.0; 64 x 64 20.9
 //              K 4096, N 16384, m = 80   36.7; 64 x 64 43.8
 //              proj, C 4096, m = 128     38.7; 64 x 64 44.4
-// K up to 1024: up to three rounds of 32 x 32, several to a CU, cost less than one of larger tiles (proj,
-// C 768, m = 160: 6.3, 64 x 64 7.8, 32 x 64 9.3; m = 256: 7.4, 64 x 64 7.8; K 768, N 3072, m = 256: 5.7, 5.5).
+// K up to 1024: two rounds of 32 x 32 (528 tiles and no more), several to a CU, cost less than one of larger
+// tiles (proj, C 768, 440 tiles: 6.9, 64 x 64 7.9, 32 x 64 7.8; 528: 7.8, 8.0; 616: 8.5, 8.1.  K 1024, N 4096, 512 tiles:
+// 6.9, 64 x 64 7.4; proj, C 1024, 560 tiles: 10.1, 8.9).
 //
 // Beyond one round of 128 x 64: 64 x 64 with four waves, two to a CU, where 128-row tiles would pad more
-// rows (K 2048, N 65536, m = 129: 101, 128 x 64 121; K 4096, N 16384, m = 160: 53, 57.5) or K is short (K 768,
-// N 65536, m = 128: 34, 38); 128 x 64 otherwise (K 4096, N 16384, m = 256: 58, 66).
+// rows (K 2048, N 65536, m = 129: 101, 128 x 64 121; K 4096, N 16384, m = 160: 53, 55.5), come to no more than one
+// and a half rounds (proj, C 2560, m = 256, 264 tiles: 35.6, 128 x 64 40.3, 64 x 64 with eight waves 38.7; K 3072, N
+// 12288, m = 256, 384 tiles: 38.4, 41.5) or K is short (K 768, N 65536, m = 128: 34, 38); 128 x 64 otherwise (proj, C 4096, m =
+// 256, 412 tiles: 61, 69; K 4096, N 16384, m = 256: 56, 66).
 //
 // K up to 512 (the low-rank outputs): a workgroup lives for one to four loads, so many small
 // ones side by side hide each other's start (four of N 2048, m = 128: 32 x 64 with four waves 4.5, 64 x 64
-// with eight 4.9; m = 256: 5.4, 9.1 with 128 x 64; N 4096, m = 128: 5.4, 9.1).
+// with eight 4.9; m = 256: 5.4, 9.1 with 128 x 64; N 4096, m = 128: 5.4, 9.1).  Up to 32 rows, where the
+// weights are all there is to load, eight waves on 32 x 32 (four of N 4096, m = 16: 4.9, 32 x 64 with four waves 5.7).
+//
+// K parts: 64 x 64 before 32 x 64 where that makes more than two fifths of the CUs' workgroups (C 768, F 3072, m = 160, three
+// parts, 108 of them: 8.1, 32 x 64 8.4; with 96 the smaller tile wins: m = 224, two parts 8.5, 7.3).
 FragConfig pick_frag_config(const FBatch& bt, int splits) {
   int max_m = 0, max_k = 0;
   int64_t kdiv = 0;  // gcd of the padded K
@@ -421,13 +428,16 @@ FragConfig pick_frag_config(const FBatch& bt, int splits) {
   const int cus = device_cus();
   auto fits = [&](int bm, int bn) { return (int64_t)tiles_for(bt, bm, bn) * splits <= cus; };
   if (fits(32, 32)) return {1, 1, 8, ks_for(8, 4)};
-  if (splits == 1 && max_k <= 512) return {1, 2, 4, 1};
-  if (splits == 1 && max_k <= 1024 && tiles_for(bt, 32, 32) <= 3 * cus) return {1, 1, 8, ks_for(8, 4)};
+  if (splits == 1 && max_k <= 512 && max_m > 32) return {1, 2, 4, 1};
+  if (splits == 1 && max_k <= 1024 && (int64_t)16 * tiles_for(bt, 32, 32) <= 33 * cus) return {1, 1, 8, ks_for(8, 4)};
+  if (splits > 1 && max_m > 64 && fits(64, 64) && 5 * tiles_for(bt, 64, 64) * splits > 2 * cus)
+    return {2, 2, 8, ks_for(8, 2)};
   if (fits(32, 64)) return {1, 2, 8, ks_for(8, 2)};
   if (fits(64, 64)) return {2, 2, 8, ks_for(8, 2)};
   if (fits(128, 64)) return {4, 2, 4, ks_for(4, 2)};
   if (max_m <= 32) return {1, 2, 8, ks_for(8, 2)};
-  if (splits == 1 && (max_k <= 1024 || tiles_for(bt, 64, 64) < 2 * tiles_for(bt, 128, 64))) return {2, 2, 4, 2};
+  const int64_t t128 = tiles_for(bt, 128, 64);
+  if (splits == 1 && (max_k <= 1024 || tiles_for(bt, 64, 64) < 2 * t128 || 2 * t128 <= 3 * cus)) return {2, 2, 4, 2};
   return {4, 2, 4, ks_for(4, 2)};
 }
 
@@ -600,6 +610,28 @@ extern "C" int vkwr_frag_gemm_f16(int n_problems, const vkwr_frag_gemm_problem* 
   }
   if (int e = launch_frag(bt, cfg, wgs, (hipStream_t)stream)) return e;
   return check_launch(fn);
+}
+
+extern "C" int vkwr_frag_gemm_f16_route(int n_problems, const vkwr_frag_gemm_problem* problems, int splits,
+                                        vkwr_frag_gemm_route* route) {
+  clear_error();
+  const char* fn = "vkwr_frag_gemm_f16_route";
+  VK_REQUIRE(n_problems >= 1 && n_problems <= kMaxFragProblems, "%s: 1..%d problems per launch (got %d)", fn,
+             kMaxFragProblems, n_problems);
+  VK_REQUIRE(problems != nullptr && route != nullptr, "%s: null pointer", fn);
+  VK_REQUIRE(splits >= 1 && splits <= 16 && (splits == 1 || n_problems == 1), "%s: bad splits (%d)", fn, splits);
+  FBatch bt;
+  bt.n = 0;
+  for (int i = 0; i < n_problems; ++i) {
+    bool empty = false;
+    if (int e = fill_problem(fn, i, problems[i], bt.p[bt.n], empty)) return e;
+    if (!empty) ++bt.n;
+  }
+  *route = vkwr_frag_gemm_route{0, 0, 0, 0};
+  if (bt.n == 0) return VKWR_OK;
+  const FragConfig c = pick_frag_config(bt, splits);
+  *route = vkwr_frag_gemm_route{32 * c.tm, 32 * c.tn, c.nw, tiles_for(bt, 32 * c.tm, 32 * c.tn) * splits};
+  return VKWR_OK;
 }
 
 extern "C" int64_t vkwr_frag_gemm_splitk_workspace_bytes(int64_t m, int64_t n, int splits) {
