@@ -102,3 +102,5 @@ def test_value_parts_of_every_batch(C):
         assert n not in (2, 4, 8) or got in (2, 4, 8), (B, got, n)
     assert {2048: [8, 8, 4, 4, 4, 2], 2560: [1, 1, 1, 2, 2, 2], 4096: [4, 4, 4, 2, 2, 1],
             1536: [2, 2, 2, 3, 3, 2]}.get(C) in (None, [parts(B) for B in (8, 64, 128, 160, 192, 300)])
+    if C == 1024:
+        assert parts(512) == 2  # (four parts of 128 x 64 would be 1024 deep: 12.2 us, two of 64 x 64 10.7)

@@ -235,7 +235,7 @@ class DecodeEngine:
 
     def _value_splits(self, B):
         """K parts of the FFN value GEMM at batch B: enough 64x64-tile parts (128x64 where 64x64 tiles
-        alone come to 96 or more and the larger ones leave more parts) to give the 256 CUs one workgroup
+        alone come to 96 or more and the larger ones leave more parts of 2048 or deeper) to give the 256 CUs one workgroup
         each, each part at least 256 deep in K.  C = 2048, B = 160: 4 parts of 128x64 18.8 us, 2 of 64x64
         20.3; C = 4096, B = 128: 36.8, 42.5.  A number of parts that the next LayerNorm adds is not given up
         for another: six layers at C = 1536, B = 300 take 748 us with 2 parts, 772 with 3 (C = 2560, B = 160,
@@ -252,7 +252,7 @@ class DecodeEngine:
         tiles, splits = parts(64)
         if tiles >= 96:
             _, wide = parts(128)
-            if wide > splits and (wide in LN_PARTS or splits not in LN_PARTS):
+            if wide > splits and (wide in LN_PARTS or splits not in LN_PARTS) and capi.frag_pad(F) >= 2048 * wide:
                 splits = wide
         return splits
 
