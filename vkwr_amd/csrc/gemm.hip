@@ -2392,9 +2392,12 @@ double big_estimate(const Batch& bt, const BigPlan& pl, double planned) {
     const double f = pl.bm == 192 ? 0.8 : 1.0;
     t = k / kBigBK * f * (0.8 + 0.9 * pl.dp_tiles / G) + 7.4;
   } else {
-    t = planned + 4.0;
+    // (nothing on top where every 256-row tile is cut in parts: M = 2100, K = 8192, N = 2048 84 us, mid-size 91; M
+    // = 680, K = 16384, N = 4096 110, 119; with whole rounds before the parts or 192-row tiles the mid-size path keeps
+    // its lead: M = 2839, K = 8192, N = 2048 104, mid-size 98)
+    t = planned + (pl.sk_tiles > 0 && pl.dp_tiles == 0 && pl.bm == 256 ? 0.0 : 4.0);
   }
-  return 1.1 * std::max(t, gemm_stream_us(bt));
+  return std::max(t, gemm_stream_us(bt)) + 0.1 * t;  // (as in mid_estimate: M = 256, N = 65536, K = 768 is 37.5 us, mid-size 39.9)
 }
 
 // Scratch that vkwr_gemm_f16_noalloc holds, and so the most partials (bytes) a mid-size plan may take.
