@@ -850,7 +850,7 @@ struct ChunkLds {
 // under a state of zeros 0 * inf would make NaN of rows that one chain keeps finite.  So every M, N,
 // q, y0 and S_start is held against kSegMax, below which no sum of steps 2 and 3 can overflow; a
 // chain with a value beyond it, or a NaN, is run token by token in step 2 instead, from the state
-// that it still has (1.25 us a token: for such inputs only).  Looking costs every call 1 - 2 us (T =
+// that it still has (1.15 us a token: for such inputs only).  Looking costs every call 1 - 2 us (T =
 // 1500: 75.4 -> 76.8); a further launch of the one-chain kernel for such chains would cost 3.
 struct SegArgs {
   int P, cps;    // segments, chunks per segment
@@ -1292,27 +1292,38 @@ __global__ __launch_bounds__(512) void wkv7_fp32_chunk_kernel(RowsArgs ra, SegAr
 
 // `len` tokens of one chain, one after the other, by 1024 threads: thread tid holds row tid / 16, columns
 // 4 (tid % 16) .. + 3 of the state S (64 x 64).  The next token's vectors are requested a token ahead.
-__device__ __forceinline__ void chain_tokens(const Fp32Args& p, float* S, size_t tok0, int len) {
+__device__ __forceinline__ void chain_tokens(const RowsArgs& ra, float* S, size_t tok0, int len) {
+  const Fp32Args& p = ra.a;
   const int tid = threadIdx.x, i = tid >> 4, j = 4 * (tid & 15);
   struct Tok {
-    _Float16 r[4], w[4], k[4], a[4], b[4], v;
+    hv4 r, w, k, a, b;
+    _Float16 v;
+  };
+  auto ld4 = [&](const _Float16* at) __attribute__((always_inline)) {
+    hv4 x;
+    if (ra.vec) {
+      x = *reinterpret_cast<const hv4*>(at);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = at[e];
+    }
+    return x;
   };
   auto fetch = [&](int t) __attribute__((always_inline)) {
     const size_t at = tok0 + (size_t)min(t, len - 1) * p.C;
-    Tok x;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      x.r[e] = p.r[at + j + e], x.w[e] = p.w[at + j + e], x.k[e] = p.k[at + j + e];
-      x.a[e] = p.a[at + j + e], x.b[e] = p.b[at + j + e];
-    }
-    x.v = p.v[at + i];
+    return Tok{ld4(p.r + at + j), ld4(p.w + at + j), ld4(p.k + at + j), ld4(p.a + at + j), ld4(p.b + at + j), p.v[at + i]};
+  };
+  // the sum over the row's 16 lanes, in each of them
+#define VK_ROW_ROR(x, n) \
+  __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + n, 0xF, 0xF, false))
+  auto sum16 = [](float x) __attribute__((always_inline)) {
+    x += VK_ROW_ROR(x, 8);
+    x += VK_ROW_ROR(x, 4);
+    x += VK_ROW_ROR(x, 2);
+    x += VK_ROW_ROR(x, 1);
     return x;
   };
-  auto sum16 = [](float x) {
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) x += __shfl_xor(x, o, 16);
-    return x;
-  };
+#undef VK_ROW_ROR
   float s[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) s[e] = S[i * kHead + j + e];
@@ -1343,7 +1354,8 @@ __device__ __forceinline__ void chain_tokens(const Fp32Args& p, float* S, size_t
 // rows 16 ri, columns 16 cj.  S goes through LDS as the next product's A operand; the next
 // segment's M and N tiles are requested before the current products.
 template <bool kSlots>
-__global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(Fp32Args p, SegArgs sg) {
+__global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(RowsArgs ra, SegArgs sg) {
+  const Fp32Args& p = ra.a;
   __shared__ __attribute__((aligned(16))) float s[kHead][kHP];
   __shared__ int apart;  // some value is beyond kSegMax
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -1399,7 +1411,7 @@ __global__ __launch_bounds__(1024) void wkv_seg_chain_kernel(Fp32Args p, SegArgs
   __syncthreads();
   if (tid == 0) sg.done[bh] = apart;
   if (apart)
-    chain_tokens(p, S, ((size_t)bi * p.T + sg.t0) * p.C + (size_t)h * kHead, sg.len);
+    chain_tokens(ra, S, ((size_t)bi * p.T + sg.t0) * p.C + (size_t)h * kHead, sg.len);
   else
     *reinterpret_cast<fq4*>(S + tid * 4) = end;
 }
@@ -1546,7 +1558,7 @@ void launch_fp32(const Fp32Args& p, int B, hipStream_t stream, bool rows, void* 
                    marks, marks + (int64_t)4 * B * p.H * s.P, rows, rows + (int64_t)B * len * p.C};
         const dim3 grid(B * p.H * sg.P);
         hipLaunchKernelGGL((wkv7_fp32_chunk_kernel<kSlots, true>), grid, dim3(512), 0, stream, ra, sg);
-        hipLaunchKernelGGL(wkv_seg_chain_kernel<kSlots>, dim3(B * p.H), dim3(1024), 0, stream, p, sg);
+        hipLaunchKernelGGL(wkv_seg_chain_kernel<kSlots>, dim3(B * p.H), dim3(1024), 0, stream, ra, sg);
         hipLaunchKernelGGL(wkv_seg_out_kernel<kSlots>, grid, dim3(256), 0, stream, p, sg);
       }
     } else if (ra.vec && B * p.H < 2 * device_cus())
