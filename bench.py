@@ -430,10 +430,10 @@ def wkv_fp16_family(dev, steps, seq_calls=20, warmup=5):
         "calls": seq_calls,
         "workload": "B=8, T=1024, H=32, fp16 state, inputs drawn as in config 0; 256 (sequence, head) "
                     "chains of 1024 dependent tokens (latency-bound: four waves per chain)",
-        "kernel": "wkv7_fp16_quad_kernel<false>: T >= 4 with at most one chain per CU"}
+        "kernel": "wkv7_fp16_quad_kernel<false>: T >= 5 with at most one chain per CU"}
     del r, w, k, v, a, b, st, yp
     torch.cuda.empty_cache()
-    out["kernel"] = ("wkv7_fp16_kernel<false> (T = 1) and wkv7_fp16_quad_kernel<false> (T >= 4, at most one chain per CU), "
+    out["kernel"] = ("wkv7_fp16_kernel<false> (T = 1) and wkv7_fp16_quad_kernel<false> (T >= 5, at most one chain per CU), "
                      "vkwr_amd/csrc/wkv.hip: one wave64 or four per (sequence, head)")
     out["timing"] = "decode: HIP graph of the steps, HIP events on the replay stream; prefill: eager calls"
     return out

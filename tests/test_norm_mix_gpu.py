@@ -232,9 +232,10 @@ def test_token_shift_prev_is_entry_value_for_long_prefill(gpu):
 
 
 @pytest.mark.parametrize("n_mix", [1, 6])
-@pytest.mark.parametrize("B,T,C", [(1, 2, 72), (2, 5, 64), (3, 4, 70), (40, 9, 2048), (130, 3, 2048), (9, 8, 24576)])
+@pytest.mark.parametrize("B,T,C", [(1, 2, 72), (2, 5, 64), (3, 4, 70), (40, 9, 2048), (130, 3, 2048), (9, 8, 24576),
+                                   (70, 5, 4096), (33, 13, 2056), (64, 7, 4096)])
 def test_token_shift_runs(gpu, n_mix, B, T, C):
-    """Runs of 2 and of 4 tokens, whole and with a remainder, vector and scalar: mix = 1 gives the
+    """Runs of 2, 3 and 4 tokens, whole and with a remainder, vector and scalar: mix = 1 gives the
     previous token and mix = 0 the token itself, exactly (values whose difference is exact)."""
     from vkwr._ops.v1 import v1_mix_ops as M
     x, shift0 = ((np.round(h(*s) * 8) / 8).clip(-4, 4).astype(np.float16) for s in ((B, T, C), (B, C)))

@@ -4,7 +4,7 @@
 // elementwise activations.  All HBM-bound.
 //
 // Token shift.  A lane owns 8 consecutive channels (one 16-byte access) of one
-// sequence for a run of 2 or 4 tokens, so x[t-1] is reused from registers.  shift_state[b] is read (the previous token at t = 0) and then
+// sequence for a run of 2 to 4 tokens, so x[t-1] is reused from registers.  shift_state[b] is read (the previous token at t = 0) and then
 // overwritten with x[b,T-1] by the same lane -- the lane whose run starts at
 // t = 0 -- so prev at t = 0 is always the value at entry.  Algorithmic bytes
 // per token and channel: 2 (x) + 2n (outputs), plus 4 per sequence and
@@ -328,8 +328,12 @@ int launch_shift(const ShiftArgs& p, bool half, const char* fn, hipStream_t s) {
   // Short runs fill the CUs and put all of a lane's rows in flight; long ones re-read less.  With
   // runs of 16 walked row by row: T = 700, C = 2048, one mix 8.3 us (TR = 4 5-8, TR = 2 7.3); T = 50, six
   // mixes 11.2 (TR = 2 4.5); 3 x 333, six mixes 13.5 (TR = 4 7.9); 8 x 1024, six mixes 38.7 (TR = 4 37.9).
-  const int64_t lanes4 = (int64_t)p.B * ((p.T + 3) / 4) * (p.C / VW);
+  // From 3 to 16 tokens, runs of 3 where those end with fewer empty places (256 sequences of C 4096, six mixes: T = 5
+  // runs of 16 15.4, of 4 16.6, of 3 15.5; T = 6 17.6, 18.3, 16.7; 128 of T = 13 18.5, 19.0, 16.9).
+  const int runs3 = (p.T + 2) / 3, runs4 = (p.T + 3) / 4;
+  const int64_t lanes4 = (int64_t)p.B * runs4 * (p.C / VW);
   if (lanes4 < 32768) return launch_shift_run<VW, NMIX, 2>(p, half, fn, s);
+  if (p.T >= 3 && p.T <= 16 && 3 * runs3 < 4 * runs4) return launch_shift_run<VW, NMIX, 3>(p, half, fn, s);
   return launch_shift_run<VW, NMIX, 4>(p, half, fn, s);
 }
 

@@ -2018,7 +2018,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   }
 }
 
-// The same recurrence for T >= 4 with at most one chain per CU and 16-byte aligned rows: four waves per (sequence,
+// The same recurrence for T >= 5 with at most one chain per CU and 16-byte aligned rows: four waves per (sequence,
 // head), so that a lone wave's 160 FMAs per token become ~90 on each of the four SIMDs.
 //
 // Wave w owns rows 16 w .. 16 w + 15; the four lanes of a quad hold one row, lane cg of it columns 16
@@ -2444,9 +2444,9 @@ static int launch_fp16(const char* fn, bool legacy, int B, int T, int C, int H, 
   const bool seq = T > 1 && (int64_t)B * H <= 4 * (int64_t)device_cus();
   // ... and four waves per chain where each has a CU to itself and the rows are 16-byte aligned: T = 300,
   // 256 chains 201 -> 117 us; two to a CU lose (288 chains 198 us with one wave, 218 with four; 512: 201, 226),
-  // and from T = 4 (8 sequences of 2 tokens 7.7 us with one wave, 8.7 with four; 2 of 4: 8.8, 8.7)
+  // and from T = 5 (8 sequences of 2 tokens, 32 heads 7.7 us with one wave, 8.7 with four; 8 of 4, in a graph, 6.1, 6.5)
   auto al = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-  const bool quad = T >= 4 && (int64_t)B * H <= (int64_t)device_cus() && al(state) && al(r) && al(w) && al(k) &&
+  const bool quad = T >= 5 && (int64_t)B * H <= (int64_t)device_cus() && al(state) && al(r) && al(w) && al(k) &&
                     al(v) && al(a) && al(b);
   if (quad) {
     if (legacy) hipLaunchKernelGGL(wkv7_fp16_quad_kernel<true>, dim3(B * H), dim3(256), 0, (hipStream_t)stream, p);
